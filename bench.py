@@ -336,7 +336,7 @@ def run_prefill_prep(lib, hip, dev, g, stream) -> dict:
     ms1 = timed(one)
     return {"prep_workload": "config 3 from fp32 projections: q/k RMSNorm + rotary + fp16 cast + append, then "
                              "causal attention, per chunk-layer",
-            "prep_entry": "ifn_paged_prefill_prep_append (one launch per chunk-layer)",
+            "prep_entry": "ifn_paged_prefill_prep_append (one call per chunk-layer)",
             "prep_fused_us_per_chunk_layer": [round(float(x), 2) for x in ms1.mean(0) * 1e3],
             "prep_fused_us_per_layer": round(float(ms1.sum(1).mean() * 1e3), 2),
             "prep_two_launch_us_per_chunk_layer": [round(float(x), 2) for x in ms2.mean(0) * 1e3],

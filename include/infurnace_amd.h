@@ -449,8 +449,8 @@ int ifn_paged_decode_prep_append(void* out, const float* q, const float* k, cons
                                  void* stream);
 
 /*
- * One prefill chunk of one layer from the fp32 projections, in one launch:
- * the pre-append of ifn_qk_norm_rope_append (q/k RMSNorm and rotary, k/v cast
+ * One prefill chunk of one layer from the fp32 projections, in one call (two
+ * launches on the stream): the pre-append of ifn_qk_norm_rope_append (q/k RMSNorm and rotary, k/v cast
  * to fp16 and stored) and the causal attention of ifn_paged_prefill over the
  * result.  Token t of the chunk has position query_start + t, for its rotary
  * angle and for its cache slot block_table[p / 16] * 16 + p % 16 (slots whose
@@ -459,8 +459,8 @@ int ifn_paged_decode_prep_append(void* out, const float* q, const float* k, cons
  * [num_q_tokens][num_kv_heads][head_dim]; the other arguments as in those two
  * calls.  `out` and the pool are bit-identical to ifn_qk_norm_rope_append(...)
  * with positions query_start + t and those slots, followed by
- * ifn_paged_prefill(...) on the fp16 query; the fp16 query itself is not
- * written.  Requires query_start % 32 == 0 (else IFN_ERR_UNSUPPORTED: run the
+ * ifn_paged_prefill(...) on the fp16 query.  The fp16 query passes through
+ * `out`, which must therefore overlap no other argument.  Requires query_start % 32 == 0 (else IFN_ERR_UNSUPPORTED: run the
  * two calls), query_start + num_q_tokens <= max_positions, every pointer
  * 16-byte aligned, and the shapes ifn_paged_prefill compiles.  Same workspace
  * as ifn_paged_prefill.

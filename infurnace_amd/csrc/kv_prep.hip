@@ -116,16 +116,18 @@ __global__ __launch_bounds__(kPrepThreads) void qk_norm_rope_append_kernel(
 // positions, then their rotary rows, before it computes.  q and k equal the
 // one-token-per-workgroup kernel's bit for bit (the same sum of squares, see PrepRows; the same
 // per-pair arithmetic), v is the same cast.
+// kChunk: the tokens are a prefill chunk's, at positions query_start + t, and their slots are those
+// positions' in the sequence's block table (`positions` is that table, slot_mapping and active are unused).
 constexpr int kPrepRowsThreads = 256;
 constexpr int kPrepPasses = 2;
 
-template <int D>
+template <int D, bool kChunk>
 __global__ __launch_bounds__(kPrepRowsThreads) void qk_norm_rope_rows_kernel(
     f16* __restrict__ q_out, const float* __restrict__ q, const float* __restrict__ k,
     const float* __restrict__ v, const float* __restrict__ q_norm_w, const float* __restrict__ k_norm_w,
     const float* __restrict__ rope, int32_t max_pos, const int32_t* __restrict__ positions,
     const int32_t* __restrict__ slot_mapping, const uint8_t* __restrict__ active, f16* __restrict__ pool,
-    int64_t num_slots, int32_t T, int32_t hq, int32_t hkv, float eps) {
+    int64_t num_slots, int32_t T, int32_t hq, int32_t hkv, float eps, int32_t query_start, int32_t block_size) {
   using PR = PrepRows<D>;
   const int lane = threadIdx.x % kWave;
   const int e = lane % PR::kLanes, sub = lane / PR::kLanes;
@@ -145,7 +147,7 @@ __global__ __launch_bounds__(kPrepRowsThreads) void qk_norm_rope_rows_kernel(
                        : head[p] < hq + hkv ? k + (int64_t(tok[p]) * hkv + (head[p] - hq)) * D
                                             : v + (int64_t(tok[p]) * hkv + (head[p] - hq - hkv)) * D;
     x[p] = load_pairs8<D>(src, e);
-    pos[p] = positions[tok[p]];
+    pos[p] = kChunk ? query_start + tok[p] : positions[tok[p]];
   }
   const Pairs8 wq = load_pairs8<D>(q_norm_w, e);
   const Pairs8 wk = load_pairs8<D>(k_norm_w, e);
@@ -172,7 +174,13 @@ __global__ __launch_bounds__(kPrepRowsThreads) void qk_norm_rope_rows_kernel(
       dst = q_out + (int64_t(t) * hq + h) * D;
       if (!pos_ok) lo = hi = u32x4{0u, 0u, 0u, 0u};
     } else {
-      const int64_t slot = slot_mapping[t];
+      int64_t slot;
+      if constexpr (kChunk) {
+        const int64_t page = positions[pos[p] / block_size];
+        slot = page * block_size + pos[p] % block_size;  // (a negative page: a negative slot)
+      } else {
+        slot = slot_mapping[t];
+      }
       if (!(pos_ok && (active == nullptr || active[t] != 0) && slot >= 0 && slot < num_slots)) continue;
       // pool layer: [2][slot][hkv][D]; V is num_slots rows after K
       dst = pool + (int64_t(kind - 1) * num_slots + slot) * hkv * D + int64_t(kind == 1 ? h - hq : h - hq - hkv) * D;
@@ -180,6 +188,24 @@ __global__ __launch_bounds__(kPrepRowsThreads) void qk_norm_rope_rows_kernel(
     *reinterpret_cast<u32x4*>(dst + 8 * e) = lo;
     *reinterpret_cast<u32x4*>(dst + D / 2 + 8 * e) = hi;
   }
+}
+
+static int64_t prep_rows_blocks(int32_t T, int32_t hq, int32_t hkv, int32_t d) {
+  const int64_t rows = int64_t(T) * (hq + 2 * hkv);
+  return ceil_div(ceil_div(rows, int64_t(kWave / (d / 16)) * kPrepPasses), kPrepRowsThreads / kWave);
+}
+
+// The pre-append of a prefill chunk (head_dim 64 or 128, 16-byte aligned arrays).
+int prep_chunk_launch(f16* q_out, const PrefillPrep& pp, int32_t max_positions, int64_t num_pages,
+                      const int32_t* block_table, int32_t query_start, int32_t T, int32_t hq, int32_t hkv, int32_t d,
+                      int32_t block_size, hipStream_t stream) {
+  const int64_t blocks = prep_rows_blocks(T, hq, hkv, d);
+  if ((d != 64 && d != 128) || blocks >= (int64_t(1) << 31)) return IFN_ERR_UNSUPPORTED;
+  auto rk = d == 128 ? qk_norm_rope_rows_kernel<128, true> : qk_norm_rope_rows_kernel<64, true>;
+  rk<<<dim3(unsigned(blocks)), dim3(kPrepRowsThreads), 0, stream>>>(
+      q_out, pp.q, pp.k, pp.v, pp.q_norm_w, pp.k_norm_w, pp.rope, max_positions, block_table, nullptr, nullptr,
+      pp.pool, num_pages * block_size, T, hq, hkv, pp.eps, query_start, block_size);
+  return ifn_launch_status();
 }
 
 // One thread block per (layer, K|V, listed page): 16-byte stores (and loads) over the page.
@@ -249,16 +275,13 @@ extern "C" int ifn_qk_norm_rope_append(void* q_out, const float* q, const float*
   auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
   if ((head_dim == 64 || head_dim == 128) && aligned(q_out) && aligned(q) && aligned(k) && aligned(v) &&
       aligned(q_norm_weight) && aligned(k_norm_weight) && aligned(rope_table) && aligned(kv_pool_layer)) {
-    const int64_t rows = int64_t(num_tokens) * (num_q_heads + 2 * num_kv_heads);
-    const int per_pass = kWave / (head_dim / 16);
-    const int64_t waves = ceil_div(rows, int64_t(per_pass) * kPrepPasses);
-    const int64_t blocks = ceil_div(waves, kPrepRowsThreads / kWave);
+    const int64_t blocks = prep_rows_blocks(num_tokens, num_q_heads, num_kv_heads, head_dim);
     if (blocks < (int64_t(1) << 31)) {
-      auto rk = head_dim == 128 ? qk_norm_rope_rows_kernel<128> : qk_norm_rope_rows_kernel<64>;
+      auto rk = head_dim == 128 ? qk_norm_rope_rows_kernel<128, false> : qk_norm_rope_rows_kernel<64, false>;
       rk<<<dim3(unsigned(blocks)), dim3(kPrepRowsThreads), 0, s>>>(
           static_cast<f16*>(q_out), q, k, v, q_norm_weight, k_norm_weight, rope_table, max_positions, positions,
           slot_mapping, active_mask, static_cast<f16*>(kv_pool_layer), num_pages * block_size, num_tokens,
-          num_q_heads, num_kv_heads, eps);
+          num_q_heads, num_kv_heads, eps, 0, block_size);
       return ifn_launch_status();
     }
   }

@@ -171,7 +171,7 @@ extern "C" int ifn_paged_prefill_prep_append(void* out, const float* q, const fl
     return IFN_ERR_INVALID_ARGUMENT;
   if (block_size != kPBlock) return IFN_ERR_UNSUPPORTED;
   if (!wide_prefill_supported(num_q_heads, num_kv_heads, head_dim)) return IFN_ERR_UNSUPPORTED;
-  if (query_start % 32 != 0) return IFN_ERR_UNSUPPORTED;  // a key tile must be wholly before or in the chunk
+  if (query_start % 32 != 0) return IFN_ERR_UNSUPPORTED;  // (the interface's requirement)
   IFN_CHECK_ALIGN16(out);
   IFN_CHECK_ALIGN16(q);
   IFN_CHECK_ALIGN16(k);
@@ -186,10 +186,22 @@ extern "C" int ifn_paged_prefill_prep_append(void* out, const float* q, const fl
   if (int64_t(query_start) + num_q_tokens > max_positions) return IFN_ERR_INVALID_ARGUMENT;  // past the table
   const int cus = device_cu_count();
   if (cus < 1) return IFN_ERR_HIP;
-  if (scale <= 0.f) scale = 1.0f / sqrtf(float(head_dim));
+  // (refused before anything is written)
+  const size_t need = wide_prefill_ws_bytes(num_q_tokens, query_start, num_q_heads, num_kv_heads, head_dim, cus);
+  if (need > 256) {
+    if (workspace == nullptr || workspace_bytes < need) return IFN_ERR_WORKSPACE;
+    IFN_CHECK_ALIGN16(workspace);
+  }
+  // The fp16 queries pass through `out`: the attention's workgroups each read their own query rows
+  // before they write them (a key split's last arrival writes after every split has read).
+  // Preparing the chunk inside the attention launch instead made every workgroup prepare the chunk
+  // tiles it reads: 16 query heads / 8 kv heads x 128, 512 tokens at 1024, 29.3 us against 22.2 us (events).
   const PrefillPrep prep{q, k, v, q_norm_weight, k_norm_weight, rope_table, static_cast<f16*>(kv_pool_layer), eps};
-  return wide_prefill_launch(static_cast<f16*>(out), nullptr, static_cast<const f16*>(kv_pool_layer), num_pages,
-                             block_table, query_start, num_q_tokens, num_q_heads, num_kv_heads, head_dim,
-                             scale * kLog2e, workspace, workspace_bytes, PrefillAppend{nullptr, nullptr, nullptr}, cus,
-                             reinterpret_cast<hipStream_t>(stream), &prep);
+  const int rc = prep_chunk_launch(static_cast<f16*>(out), prep, max_positions, num_pages, block_table, query_start,
+                                   num_q_tokens, num_q_heads, num_kv_heads, head_dim, block_size,
+                                   reinterpret_cast<hipStream_t>(stream));
+  if (rc != IFN_OK) return rc;
+  return prefill_entry(out, out, kv_pool_layer, num_pages, block_table, max_pages, query_start, num_q_tokens,
+                       num_q_heads, num_kv_heads, head_dim, block_size, scale, workspace, workspace_bytes, stream,
+                       PrefillAppend{nullptr, nullptr, nullptr});
 }

@@ -28,10 +28,6 @@
 //    lazy rescale of the running maximum (slack 2^8); row sums add the fp16 probabilities.
 //  * Epilogue: the W key groups merge log-sum-exp style through LDS, each wave finishing its share
 //    of the output; then the key-split merge and the fp16 stores.
-//  * Fused pre-append (kPrep): the chunk's queries, keys and values arrive as fp32 projections.
-//    Each wave first normalises, rotates and casts the K and V rows of the chunk tiles it will
-//    read and writes them to the pool, and the workgroup prepares its own queries straight into the
-//    LDS staging; the attention then runs as in the plain kernel.
 #include "ifn_common.hpp"
 #include "decode_rows.hpp"
 
@@ -196,12 +192,11 @@ __device__ __forceinline__ void pin_probs(f16x8 (&p)[RT][2]) {
 // The kernel's body, run by workgroup bid of grid, with its LDS at smem (WideCfg::kLdsBytes).
 // kPrefix: the caller runs only the shared-prefix pass (px.key_len > 0), so the causal limits are
 // compiled out (in the one-launch shared-prefix kernel this keeps the loop within its registers).
-template <int D, int G, int RT, int W, bool kAppend, bool kPrep, bool kPrefix = false>
+template <int D, int G, int RT, int W, bool kAppend, bool kPrefix = false>
 __device__ __forceinline__ void prefill_wide_body(
     unsigned char* smem, const int bid, const int grid, f16* out, const f16* q, const f16* pool, int64_t num_pages,
     const int32_t* table, int32_t query_start, int32_t T, int32_t num_kv_heads, int32_t n_qb, int32_t nsplit,
-    float scale_log2, PrefillWorkspace ws, PrefillAppend ap, PrefixOut px, PrefillPrep pp) {
-  static_assert(!(kAppend && kPrep), "one form of the fused append");
+    float scale_log2, PrefillWorkspace ws, PrefillAppend ap, PrefixOut px) {
   using C = WideCfg<D, G, RT, W>;
   constexpr int kKS = C::kKSteps;
   constexpr int kDT = C::kDT;
@@ -242,9 +237,7 @@ __device__ __forceinline__ void prefill_wide_body(
   const int64_t tok_stride = int64_t(num_kv_heads) * D;
   const int64_t v_off = num_pages * kWBlock * tok_stride;
   const int64_t page_elems = int64_t(kWBlock) * tok_stride;
-  // (kPrep: the pool is read through the pointer it is written through, so no read is assumed to
-  // be independent of the pre-append's stores)
-  const f16* head_pool = (kPrep ? static_cast<const f16*>(pp.pool) : pool) + int64_t(kvh) * D;
+  const f16* head_pool = pool + int64_t(kvh) * D;
 
   if constexpr (kAppend)
     wide_store_chunk(ap.pool, num_pages, table, query_start, T, num_kv_heads, D, ap.new_k, ap.new_v,
@@ -290,91 +283,12 @@ __device__ __forceinline__ void prefill_wide_body(
   // chunk as zeros), for the LDS staging below.
   lds_u8* const qlds = (lds_u8*)(smem) + C::kTileBytes;
   u32x4 qst[C::kQInstr];
-  if constexpr (!kPrep) {
 #pragma unroll
-    for (int n = 0; n < C::kQInstr; ++n) {
-      const int slot = n * kWave + lane, rho = C::kQRowsPerWave * grp + slot / C::kRowChunks, c = slot % C::kRowChunks;
-      const int qi = q0 + rho % kQw;
-      const u32x4 v = ld16(q + (int64_t(min(qi, T - 1)) * hq + kvh * G + rho / kQw) * D + 8 * c);
-      qst[n] = qi < T ? v : u32x4{0u, 0u, 0u, 0u};
-    }
-  } else {
-    using PR = PrepRows<D>;
-    const int e = lane % PR::kLanes, sub = lane / PR::kLanes;
-    // (1) This wave's tiles of the chunk (keys at or past query_start; query_start % 32 == 0): K
-    // normalised and rotated, V cast, both written to the pool at the table's slots.  Rows past the
-    // chunk and rows of an invalid page are not written (the attention reads zeros there).  The
-    // work is a list of jobs (one wave pass of kRows rows each): the wave's tiles from the first one
-    // in the chunk on (tile_of is increasing), kWTile / kRows jobs per tile.  A job's loads are
-    // issued one job ahead, before the previous job's arithmetic and stores.  The queries' loads go
-    // first, so they are in flight meanwhile.
-    constexpr int kOps = kWTile / PR::kRows;
-    const int first_tile = split * W + grp, tile_step = W * nsplit;  // tile_of(i) = first_tile + i tile_step
-    const int qs_tile = query_start / kWTile;
-    const int i0 = qs_tile > first_tile ? int(ceil_div(qs_tile - first_tile, tile_step)) : 0;
-    const int nj = iters > i0 ? (iters - i0) * kOps : 0;
-    struct Job {
-      Pairs8 k, v, cs;
-      int page;
-    };
-    auto job_pos = [&](int j) __attribute__((always_inline)) {  // key position of this lane's row of job j
-      return tile_of(i0 + j / kOps) * kWTile + (j % kOps) * PR::kRows + sub;
-    };
-    auto job_load = [&](int j) __attribute__((always_inline)) -> Job {
-      const int tc = min(job_pos(min(j, nj - 1)) - query_start, T - 1);  // (past the list: a valid row again)
-      const int64_t src = (int64_t(tc) * num_kv_heads + kvh) * D;
-      return Job{load_pairs8<D>(pp.k + src, e), load_pairs8<D>(pp.v + src, e),
-                 load_pairs8<D>(pp.rope + int64_t(query_start + tc) * D, e), table[(query_start + tc) / kWBlock]};
-    };
-    // the queries' inputs (step 2)
-    constexpr int kQOps = (C::kQRowsPerWave + PR::kRows - 1) / PR::kRows;
-    Pairs8 xq[kQOps], csq[kQOps];
-#pragma unroll
-    for (int op = 0; op < kQOps; ++op) {
-      const int rho = C::kQRowsPerWave * grp + min(op * PR::kRows + sub, C::kQRowsPerWave - 1);
-      const int qc = min(q0 + rho % kQw, T - 1);
-      xq[op] = load_pairs8<D>(pp.q + (int64_t(qc) * hq + kvh * G + rho / kQw) * D, e);
-      csq[op] = load_pairs8<D>(pp.rope + int64_t(query_start + qc) * D, e);
-    }
-    const Pairs8 wk = load_pairs8<D>(pp.k_norm_w, e);
-    if (nj > 0) {
-      Job cur = job_load(0);
-      for (int j = 0; j < nj; ++j) {
-        const Job nxt = job_load(j + 1);
-        const int pos = job_pos(j);
-        u32x4 klo, khi;
-        norm_rope_row<D>(cur.k, wk, cur.cs, pp.eps, klo, khi);
-        if (pos - query_start < T && cur.page >= 0 && int64_t(cur.page) < num_pages) {
-          f16* kd = pp.pool + (int64_t(cur.page) * kWBlock + pos % kWBlock) * tok_stride + int64_t(kvh) * D;
-          f16* vd = kd + v_off;
-          *reinterpret_cast<u32x4*>(kd + 8 * e) = klo;
-          *reinterpret_cast<u32x4*>(kd + D / 2 + 8 * e) = khi;
-          *reinterpret_cast<u32x4*>(vd + 8 * e) = pack_f16x8(cur.v.a[0], cur.v.a[1]);
-          *reinterpret_cast<u32x4*>(vd + D / 2 + 8 * e) = pack_f16x8(cur.v.b[0], cur.v.b[1]);
-        }
-        cur = nxt;
-      }
-    }
-    // (2) The workgroup's queries, normalised and rotated into the LDS staging (chunk c of row rho
-    // at c ^ (rho % 8)); wave grp prepares rows kQRowsPerWave grp .. (a row past the chunk as zeros).
-    const Pairs8 wq = load_pairs8<D>(pp.q_norm_w, e);
-#pragma unroll
-    for (int op = 0; op < kQOps; ++op) {
-      const int rw = op * PR::kRows + sub;
-      const int rho = C::kQRowsPerWave * grp + min(rw, C::kQRowsPerWave - 1);
-      const int qi = q0 + rho % kQw;
-      u32x4 lo, hi;
-      norm_rope_row<D>(xq[op], wq, csq[op], pp.eps, lo, hi);
-      if (qi >= T) lo = hi = u32x4{0u, 0u, 0u, 0u};
-      if (rw < C::kQRowsPerWave) {
-        *reinterpret_cast<__attribute__((address_space(3))) u32x4*>(qlds + rho * 2 * D + ((e ^ (rho % 8)) * 16)) = lo;
-        *reinterpret_cast<__attribute__((address_space(3))) u32x4*>(
-            qlds + rho * 2 * D + (((PR::kLanes + e) ^ (rho % 8)) * 16)) = hi;
-      }
-    }
-    // The pool stores are complete before any of this wave's K or V requests (it reads back only
-    // rows it wrote itself; the memory clobber keeps the compiler from hoisting them).
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  for (int n = 0; n < C::kQInstr; ++n) {
+    const int slot = n * kWave + lane, rho = C::kQRowsPerWave * grp + slot / C::kRowChunks, c = slot % C::kRowChunks;
+    const int qi = q0 + rho % kQw;
+    const u32x4 v = ld16(q + (int64_t(min(qi, T - 1)) * hq + kvh * G + rho / kQw) * D + 8 * c);
+    qst[n] = qi < T ? v : u32x4{0u, 0u, 0u, 0u};
   }
   // The window arrives before the first tiles' K and V are requested.
   asm volatile("" ::"v"(win_k.ids) : "memory");
@@ -430,9 +344,7 @@ __device__ __forceinline__ void prefill_wide_body(
       // (page and key count are uniform; readfirstlane keeps the descriptor in scalar registers)
       const bool ok = ((fl >> h) & 1) != 0;
       const int page = __builtin_amdgcn_readfirstlane(ok ? (h == 0 ? pa : pb) : 0);
-      // (kPrep: keys from key_end on -- hidden from every row here -- read as zeros, so a tile this
-      // wave did not prepare is never read)
-      const int keys = __builtin_amdgcn_readfirstlane(ok ? min(max((kPrep ? key_end : total) - (kt + 16 * h), 0), 16) : 0);
+      const int keys = __builtin_amdgcn_readfirstlane(ok ? min(max(total - (kt + 16 * h), 0), 16) : 0);
       t.r[h] = __builtin_amdgcn_make_buffer_rsrc(const_cast<f16*>(head_pool + base + int64_t(page) * page_elems), 0,
                                                  keys * int(tok_stride) * 2, 0x00020000);
       t.add[h] = 0;
@@ -746,13 +658,10 @@ __device__ __forceinline__ void prefill_wide_body(
 #pragma unroll
     for (int j = 0; j < C::kVInstr; ++j) vst[j] = v_load(v_tile(0, p0), j);
     // Q through LDS: Q^T as the B operand, K-step s = dims 16 s + 8 half .. + 7 of row 32 rt + col
-    // (kPrep: the staging is written already)
-    if constexpr (!kPrep) {
 #pragma unroll
-      for (int n = 0; n < C::kQInstr; ++n) {
-        const int slot = n * kWave + lane, rho = C::kQRowsPerWave * grp + slot / C::kRowChunks, c = slot % C::kRowChunks;
-        *reinterpret_cast<__attribute__((address_space(3))) u32x4*>(qlds + rho * 2 * D + ((c ^ (rho % 8)) * 16)) = qst[n];
-      }
+    for (int n = 0; n < C::kQInstr; ++n) {
+      const int slot = n * kWave + lane, rho = C::kQRowsPerWave * grp + slot / C::kRowChunks, c = slot % C::kRowChunks;
+      *reinterpret_cast<__attribute__((address_space(3))) u32x4*>(qlds + rho * 2 * D + ((c ^ (rho % 8)) * 16)) = qst[n];
     }
     __syncthreads();
 #pragma unroll
@@ -992,28 +901,23 @@ __device__ __forceinline__ void prefill_wide_body(
   }
 }
 
-template <int D, int G, int RT, int W, bool kAppend, bool kPrep>
+template <int D, int G, int RT, int W, bool kAppend>
 __global__ __launch_bounds__(W * kWave) void prefill_wide_kernel(
-    f16* __restrict__ out, const f16* __restrict__ q, const f16* __restrict__ pool, int64_t num_pages,
-    const int32_t* __restrict__ table, int32_t query_start, int32_t T, int32_t num_kv_heads, int32_t n_qb,
-    int32_t nsplit, float scale_log2, PrefillWorkspace ws, PrefillAppend ap, PrefixOut px, PrefillPrep pp) {
+    f16* out, const f16* q, const f16* __restrict__ pool, int64_t num_pages, const int32_t* __restrict__ table,
+    int32_t query_start, int32_t T, int32_t num_kv_heads, int32_t n_qb, int32_t nsplit, float scale_log2, PrefillWorkspace ws, PrefillAppend ap, PrefixOut px) {
   __shared__ __attribute__((aligned(16))) unsigned char smem[WideCfg<D, G, RT, W>::kLdsBytes];
-  prefill_wide_body<D, G, RT, W, kAppend, kPrep>(smem, int(blockIdx.x), int(gridDim.x), out, q, pool, num_pages, table,
-                                                 query_start, T, num_kv_heads, n_qb, nsplit, scale_log2, ws, ap, px, pp);
+  prefill_wide_body<D, G, RT, W, kAppend>(smem, int(blockIdx.x), int(gridDim.x), out, q, pool, num_pages, table,
+                                          query_start, T, num_kv_heads, n_qb, nsplit, scale_log2, ws, ap, px);
 }
 
 typedef void (*WideKernel)(f16*, const f16*, const f16*, int64_t, const int32_t*, int32_t, int32_t, int32_t, int32_t,
-                           int32_t, float, PrefillWorkspace, PrefillAppend, PrefixOut, PrefillPrep);
-
-enum class WideMode { kPlain, kAppend, kPrep };
+                           int32_t, float, PrefillWorkspace, PrefillAppend, PrefixOut);
 
 // (row tiles and waves: 2 and 4 for every shape; 1 and 8 for head dim 128)
-static WideKernel pick_wide(int d, int g, int rt, int w, WideMode mode) {
+static WideKernel pick_wide(int d, int g, int rt, int w, bool append) {
 #define IFN_WIDE_CASE(DD, GG, RR, WW)                                                                \
   if (d == DD && g == GG && rt == RR && w == WW)                                                     \
-    return mode == WideMode::kAppend ? prefill_wide_kernel<DD, GG, RR, WW, true, false>              \
-           : mode == WideMode::kPrep ? prefill_wide_kernel<DD, GG, RR, WW, false, true>              \
-                                     : prefill_wide_kernel<DD, GG, RR, WW, false, false>;
+    return append ? prefill_wide_kernel<DD, GG, RR, WW, true> : prefill_wide_kernel<DD, GG, RR, WW, false>;
   IFN_WIDE_CASE(64, 1, 2, 4) IFN_WIDE_CASE(64, 2, 2, 4) IFN_WIDE_CASE(64, 4, 2, 4) IFN_WIDE_CASE(64, 8, 2, 4)
   IFN_WIDE_CASE(128, 1, 2, 4) IFN_WIDE_CASE(128, 2, 2, 4) IFN_WIDE_CASE(128, 4, 2, 4) IFN_WIDE_CASE(128, 8, 2, 4)
   IFN_WIDE_CASE(128, 1, 1, 8) IFN_WIDE_CASE(128, 2, 1, 8) IFN_WIDE_CASE(128, 4, 1, 8) IFN_WIDE_CASE(128, 8, 1, 8)
@@ -1022,7 +926,7 @@ static WideKernel pick_wide(int d, int g, int rt, int w, WideMode mode) {
 }
 
 bool wide_prefill_supported(int32_t hq, int32_t hkv, int32_t d) {
-  return hkv >= 1 && hq % hkv == 0 && pick_wide(d, hq / hkv, 2, 4, WideMode::kPlain) != nullptr;
+  return hkv >= 1 && hq % hkv == 0 && pick_wide(d, hq / hkv, 2, 4, false) != nullptr;
 }
 
 size_t wide_prefill_ws_bytes(int32_t T, int32_t query_start, int32_t hq, int32_t hkv, int32_t d, int cus) {
@@ -1032,12 +936,10 @@ size_t wide_prefill_ws_bytes(int32_t T, int32_t query_start, int32_t hq, int32_t
 int wide_prefill_launch(f16* out, const f16* q, const f16* pool, int64_t num_pages, const int32_t* table,
                         int32_t query_start, int32_t T, int32_t hq, int32_t hkv, int32_t d, float scale_log2,
                         void* workspace, size_t workspace_bytes, const PrefillAppend& ap, int cus,
-                        hipStream_t stream, const PrefillPrep* prep) {
+                        hipStream_t stream) {
   const WidePlan p = plan_wide(T, query_start, hq, hkv, d, cus);
-  const WideMode mode = prep != nullptr ? WideMode::kPrep : ap.pool != nullptr ? WideMode::kAppend : WideMode::kPlain;
-  WideKernel k = pick_wide(d, hq / hkv, p.rt, p.w, mode);
+  WideKernel k = pick_wide(d, hq / hkv, p.rt, p.w, ap.pool != nullptr);
   if (k == nullptr) return IFN_ERR_UNSUPPORTED;
-  if (prep != nullptr && (ap.pool != nullptr || query_start % kWTile != 0)) return IFN_ERR_UNSUPPORTED;
   if (p.n_qb * hkv * p.nsplit > int64_t(1) << 31) return IFN_ERR_UNSUPPORTED;
   // (the fused append indexes the chunk's K and V rows with 32-bit byte offsets)
   if (ap.pool != nullptr && int64_t(T) * hkv * d * 2 >= int64_t(1) << 31) return IFN_ERR_UNSUPPORTED;
@@ -1052,7 +954,7 @@ int wide_prefill_launch(f16* out, const f16* q, const f16* pool, int64_t num_pag
   }
   k<<<dim3(unsigned(p.n_qb * hkv * p.nsplit)), dim3(unsigned(p.w * kWave)), 0, stream>>>(
       out, q, pool, num_pages, table, query_start, T, hkv, int(p.n_qb), p.nsplit, scale_log2, ws, ap,
-      PrefixOut{nullptr, nullptr, 0, 0, nullptr}, prep != nullptr ? *prep : PrefillPrep{});
+      PrefixOut{nullptr, nullptr, 0, 0, nullptr});
   return ifn_launch_status();
 }
 
@@ -1065,13 +967,13 @@ int wide_prefix_pass(const f16* q, const f16* pool, int64_t num_pages, const int
                      f16* px_oh, int32_t stride, int cus, hipStream_t stream) {
   if (key_len < 1) return IFN_ERR_INVALID_ARGUMENT;
   const WidePlan p = plan_wide(batch, 0, hq, hkv, d, cus, key_len);
-  WideKernel k = pick_wide(d, hq / hkv, p.rt, p.w, WideMode::kPlain);
+  WideKernel k = pick_wide(d, hq / hkv, p.rt, p.w, false);
   if (k == nullptr) return IFN_ERR_UNSUPPORTED;
   if (p.n_qb * hkv * p.nsplit > int64_t(1) << 31 || stride < p.nsplit) return IFN_ERR_UNSUPPORTED;
   k<<<dim3(unsigned(p.n_qb * hkv * p.nsplit)), dim3(unsigned(p.w * kWave)), 0, stream>>>(
       nullptr, q, pool, num_pages, prefix_pages, 0, batch, hkv, int(p.n_qb), p.nsplit, scale_log2,
       PrefillWorkspace{nullptr, nullptr, nullptr}, PrefillAppend{nullptr, nullptr, nullptr},
-      PrefixOut{px_ml, px_o, key_len, stride, px_oh}, PrefillPrep{});
+      PrefixOut{px_ml, px_o, key_len, stride, px_oh});
   return ifn_launch_status();
 }
 
@@ -1139,10 +1041,10 @@ __global__ __launch_bounds__(8 * kWave) void shared_prefix_fused_kernel(
 
   // The prefix pass for (query block qb, kv head bid % Hkv, key split): its states, stored at the
   // device coherence point.
-  prefill_wide_body<D, G, 1, 8, false, false, true>(
+  prefill_wide_body<D, G, 1, 8, false, true>(
       smem, bid, npre, out, q, pool, num_pages, prefix_pages, 0, batch, HKV, n_qb, nsplit, scale_log2,
       PrefillWorkspace{nullptr, nullptr, nullptr}, PrefillAppend{nullptr, nullptr, nullptr},
-      PrefixOut{px.ml, px.o, pk, px.nstates, const_cast<f16*>(px.oh)}, PrefillPrep{});
+      PrefixOut{px.ml, px.o, pk, px.nstates, const_cast<f16*>(px.oh)});
   wait_all_mem();   // this wave's state stores acknowledged
   __syncthreads();  // ... and every other wave's; the tile buffers are free
   // The decode role's split of the rows' own keys (the same offsets and ranges), to find where a

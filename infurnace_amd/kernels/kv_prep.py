@@ -244,14 +244,14 @@ def qk_norm_rope_append_and_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.T
                                     block_table: torch.Tensor, *, query_start: int, layer: int = 0,
                                     eps: float = 1e-6, scale: float | None = None, out: torch.Tensor | None = None,
                                     block_size: int = 16, validate: bool = False) -> torch.Tensor:
-    """A prefill chunk of one layer from fp32 projections: pre-append and attention in one launch.
+    """A prefill chunk of one layer from fp32 projections: pre-append and attention in one call.
 
     ``ifn_paged_prefill_prep_append``: the same ``out`` and pool as ``qk_norm_rope_append(q, k, v,
     ..., positions, slots, None, kv_pool, layer=layer, eps=eps)`` with positions query_start + t and
     their slots in ``block_table``, followed by ``paged_attention(q16, kv_pool, block_table, None,
     None, query_start=query_start)`` -- the norm / rope / attention / cache write of a prefill
-    chunk, model.py:109-138.  q fp32 [T, Hq, D], k / v fp32 [T, Hkv, D].  A chunk the fused kernel
-    does not take (query_start not a multiple of 32, an unaligned input) runs the two launches
+    chunk, model.py:109-138.  q fp32 [T, Hq, D], k / v fp32 [T, Hkv, D].  A chunk that entry point
+    does not take (query_start not a multiple of 32, an unaligned input) goes through the two calls
     instead.  ``validate``: every table entry the chunk's keys use names a page of the pool
     (checked before the launch; a debug mode that synchronises).
     """

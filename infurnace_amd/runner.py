@@ -121,9 +121,7 @@ class _Step:
         """The same from fp32 projections: q/k RMSNorm + rotary, fp16 cast and append.
 
         A decode step without a shared prefix does all of it and the attention in one launch
-        (``qk_norm_rope_store_and_decode``); otherwise the pre-append is its own launch.  (A prefill
-        chunk keeps two launches: ``qk_norm_rope_append_and_prefill`` does it in one, but every
-        workgroup then prepares the chunk rows it reads itself, which measures slower.)
+        (``qk_norm_rope_store_and_decode``); otherwise the pre-append is its own launch.
         """
         if self.closed:
             raise RunnerError("this step is closed: a later step has begun")
