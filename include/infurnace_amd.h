@@ -355,7 +355,7 @@ int ifn_paged_decode_shared_prefix_planned(void* out, const void* query, const v
  * fp16) at slot block_table[p / 16] * 16 + p % 16 for p = query_start + t
  * (skipped where that page id is outside the pool, as ifn_store_kv skips
  * such slots), then ifn_paged_prefill(...) on the same stream.  With
- * query_start % 32 == 0 this is one launch in which the attention takes the
+ * query_start % 32 == 0 (a multiple of 16 for chunks that fill the chip) this is one launch in which the attention takes the
  * chunk's keys from new_k / new_v; otherwise the store and the attention are
  * two launches.  Same workspace as ifn_paged_prefill.
  * Replaces: store_kv then paged_attention of one prefill chunk

@@ -399,6 +399,12 @@ int wide_prefill_launch(f16* out, const f16* q, const f16* pool, int64_t num_pag
                         int32_t query_start, int32_t T, int32_t hq, int32_t hkv, int32_t d, float scale_log2,
                         void* workspace, size_t workspace_bytes, const PrefillAppend& ap, int cus,
                         hipStream_t stream);
+// Chunks whose rows fill the chip in 128-row workgroups (paged_prefill_block.hip): key groups per
+// workgroup for these shapes, 0 where the wide kernel takes them.
+int prefill_block_groups(int32_t T, int32_t query_start, int32_t hq, int32_t hkv, int32_t d, int cus);
+int prefill_block_launch(f16* out, const f16* q, const f16* pool, int64_t num_pages, const int32_t* table,
+                         int32_t query_start, int32_t T, int32_t hq, int32_t hkv, int32_t d, float scale_log2,
+                         int groups, const PrefillAppend& ap, hipStream_t stream);
 // The shared-prefix pass on that kernel (same contract as prefix_pass / prefix_pass_splits).
 int wide_prefix_splits(int32_t batch, int32_t hq, int32_t hkv, int32_t d, int32_t key_len, int cus);
 int wide_prefix_pass(const f16* q, const f16* pool, int64_t num_pages, const int32_t* prefix_pages, int32_t key_len,

@@ -6,14 +6,15 @@
 // semantics are src/infurnace/executor/tinygrad/model.py:116-132: query row i sits at
 // start_position + i and sees keys with key_pos <= query_pos.
 //
-// The attention itself is prefill_wide_kernel (paged_prefill_wide.hip): MFMA fp16 tiles, K through
-// LDS, V through transposing LDS reads.  It compiles head_dim 64 and 128 with GQA groups 1, 2, 4
-// and 8; other shapes return IFN_ERR_UNSUPPORTED.  The shared-prefix pass of the shared-prefix
+// The attention itself is prefill_wide_kernel (paged_prefill_wide.hip) or, for chunks whose rows fill
+// the chip, prefill_block_kernel (paged_prefill_block.hip): MFMA fp16 tiles, K through LDS, V through
+// transposing LDS reads.  head_dim 64 and 128 with GQA groups 1, 2, 4 and 8; other shapes return
+// IFN_ERR_UNSUPPORTED.  The shared-prefix pass of the shared-prefix
 // decode entry point runs on the same kernel (wide_prefix_pass).
 //
 // ifn_paged_prefill_append fuses the chunk's K/V store into the attention launch when
-// query_start % 32 == 0 (a key tile is then wholly before the chunk or wholly in it) and the chunk
-// fits one buffer resource; otherwise store_chunk_kernel stores the rows and the plain attention
+// query_start is a multiple of 32, or of the page on the block kernel (a key tile, or page, is then
+// wholly before the chunk or wholly in it), and the chunk fits one buffer resource; otherwise store_chunk_kernel stores the rows and the plain attention
 // follows on the same stream, with the same result.
 #include "ifn_common.hpp"
 
@@ -110,7 +111,9 @@ static int prefill_entry(void* out, const void* query, const void* kv_pool_layer
     return IFN_ERR_INVALID_ARGUMENT;  // keys past the end of the block table
   const int cus = device_cu_count();
   if (cus < 1) return IFN_ERR_HIP;
-  if (append && (query_start % 32 != 0 ||
+  if (scale <= 0.f) scale = 1.0f / sqrtf(float(head_dim));
+  const int groups = prefill_block_groups(num_q_tokens, query_start, num_q_heads, num_kv_heads, head_dim, cus);
+  if (append && (query_start % (groups > 0 ? kPBlock : 32) != 0 ||
                  int64_t(num_q_tokens) * num_kv_heads * head_dim * 2 >= (int64_t(1) << 31))) {
     // not fusable: the store as its own launch, then the plain attention (same result)
     const int64_t items = int64_t(num_q_tokens) * 2 * num_kv_heads * head_dim / 8;
@@ -121,7 +124,11 @@ static int prefill_entry(void* out, const void* query, const void* kv_pool_layer
     if (rc != IFN_OK) return rc;
     ap = PrefillAppend{nullptr, nullptr, nullptr};
   }
-  if (scale <= 0.f) scale = 1.0f / sqrtf(float(head_dim));
+  if (groups > 0)
+    return prefill_block_launch(static_cast<f16*>(out), static_cast<const f16*>(query),
+                                static_cast<const f16*>(kv_pool_layer), num_pages, block_table, query_start,
+                                num_q_tokens, num_q_heads, num_kv_heads, head_dim, scale * kLog2e, groups, ap,
+                                reinterpret_cast<hipStream_t>(stream));
   return wide_prefill_launch(static_cast<f16*>(out), static_cast<const f16*>(query),
                              static_cast<const f16*>(kv_pool_layer), num_pages, block_table, query_start,
                              num_q_tokens, num_q_heads, num_kv_heads, head_dim, scale * kLog2e, workspace,
