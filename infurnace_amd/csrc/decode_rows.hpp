@@ -95,6 +95,7 @@ constexpr int kPlanHdr = 16;
 constexpr int kPlanRec = 128;
 constexpr int kPlanPieces = 3;
 constexpr int kPlanIds = 64;
+constexpr int kPlanIdWord = 64;  // a record's first page id; words past its pieces are zero up to here
 static inline __host__ __device__ int64_t plan_rec0(int32_t batch) { return (kPlanHdr + batch + 1 + 63) / 64 * 64; }
 static inline size_t plan_words(int32_t batch, int blocks) { return size_t(plan_rec0(batch) + int64_t(blocks) * kPlanRec); }
 
@@ -257,7 +258,10 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(
     plan[6] = cap;
     plan[7] = pk;
   }
-  for (int i = tid; i <= batch; i += kPlanThreads) plan[kPlanHdr + i] = s_cum[i];
+  // (every word of the plan is written, so that a buffer needs no clearing and two plans compare equal)
+  if (tid >= 8 && tid < kPlanHdr) plan[tid] = 0;
+  for (int i = kPlanHdr + tid; i < plan_rec0(batch); i += kPlanThreads)
+    plan[i] = i <= kPlanHdr + batch ? s_cum[i - kPlanHdr] : 0;
   int32_t* recs = plan + plan_rec0(batch);
   for (int r = tid; r < nb; r += kPlanThreads) {
     int32_t* rec = recs + int64_t(r) * kPlanRec;
@@ -299,6 +303,7 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(
       }
     }
     rec[0] = n;
+    for (int w = 1 + 6 * min(n, kPlanPieces); w < kPlanIdWord; ++w) rec[w] = 0;
     s_p0[0][r] = p0b;
     s_p0[1][r] = p0a;
     s_p0[2][r] = p0e;
@@ -763,7 +768,9 @@ __device__ __forceinline__ void decode_rows_body(
       pout[6] = cap;
       pout[7] = pk;
     }
-    for (int i = tid; i <= batch; i += kRowsThreads) pout[kPlanHdr + i] = s_cum[i];
+    if (tid >= 8 && tid < kPlanHdr) pout[tid] = 0;
+    for (int i = kPlanHdr + tid; i < plan_rec0(batch); i += kRowsThreads)
+      pout[i] = i <= kPlanHdr + batch ? s_cum[i - kPlanHdr] : 0;
   }
   auto ensure_cum = [&]() __attribute__((always_inline)) {  // planned: s_cum valid after the next barrier
     if (!have_cum) {
@@ -777,7 +784,7 @@ __device__ __forceinline__ void decode_rows_body(
   // range may still hold no key (only virtual positions); it then has no piece and takes no ticket.
   const int64_t nr = range_count(nb, T);
   if (blk >= nr) {
-    if (prec != nullptr && tid <= kPlanIds) prec[tid == kPlanIds ? 0 : kPlanIds + tid] = 0;  // no piece
+    if (prec != nullptr && tid < kPlanRec) prec[tid] = 0;  // no piece
     finish();
     return;
   }
@@ -1178,7 +1185,8 @@ __device__ __forceinline__ void decode_rows_body(
 
   if (prec != nullptr) {
     if (tid == 0) prec[0] = npieces;
-    if (npieces == 0 && tid < kPlanIds) prec[kPlanIds + tid] = 0;  // (only virtual positions)
+    if (tid > 6 * min(npieces, kPlanPieces) && tid < kPlanIdWord) prec[tid] = 0;
+    if (npieces == 0 && tid < kPlanIds) prec[kPlanIdWord + tid] = 0;  // (only virtual positions)
   }
   if (!kFused && pend_n > 0) {
     // Tickets for the range's split rows: every partial store of the workgroup acknowledged first.
