@@ -163,7 +163,9 @@ int ifn_paged_decode_append(void* out, const void* query, void* kv_pool_layer, i
  * start each workgroup's page loads one round trip after launch instead of
  * three.  A plan is valid for calls with exactly the inputs it was built
  * from; it holds no pointers, so it may be built on one stream and used on
- * another once ordered after it.  plan_bytes == 0 means these shapes decode
+ * another once ordered after it.  For token rows (num_kv_heads x head_dim fp16)
+ * below 2 KiB a missing, short or unaligned plan buffer means no plan rather
+ * than an error.  plan_bytes == 0 means these shapes decode
  * without a plan (the planned entry points then ignore it).  slot_mapping may
  * be NULL for a plan used only by ifn_paged_decode_planned; a plan used by
  * ifn_paged_decode_append_planned must be built with the step's slots (else

@@ -1,5 +1,6 @@
 // Paged GQA decode over whole token rows (gfx950), for pools whose token row -- num_kv_heads x
-// head_dim fp16 -- is 2 KiB: Qwen3-0.6B and Qwen3-8B (8 KV heads x 128), and 4 x 256 / 16 x 64.
+// head_dim fp16 -- is 2 KiB: Qwen3-0.6B and Qwen3-8B (8 KV heads x 128), and 4 x 256 / 16 x 64; and for
+// 1 KiB and 512 B rows (their tensor-parallel shards, 4 and 2 heads x 128, and 8 x 64).
 //
 // Replaces the reference's documented paged_attention for decode
 // (docs/architecture.md:246; placeholder src/infurnace/kernels/paged_attention.py) whose contiguous
@@ -25,6 +26,11 @@
 //    col + 64 / Hkv of its head, so each load instruction reads 1 KiB in 128-byte runs.  The wave
 //    keeps an S-stage register ring of tokens in flight; page ids sit one per lane (64 per
 //    window) and are read with v_readlane.
+//    Of smaller token rows a wave holds TPW = 2 KiB / row size consecutive ones, each in 64 / TPW lanes
+//    with its own softmax state (8 TPW states per piece), so a load instruction still reads 1 KiB in
+//    128-byte runs.  Against the per-head kernel, which reads such rows in 256-byte pieces (planned, us):
+//    4 kv heads, 48 rows of 100-4000 keys 57.1 -> 43.8; 2 kv heads, 32 such rows 39.0 -> 23.1; 8 x 64, 40
+//    rows of 64-2000 25.4 -> 23.2; one row of 4000 keys, 4 kv heads, 54.0 -> 26.2.
 //  * q.k uses v_dot2_f32_f16 (fp32 accumulation) and a DPP reduction over the head's lanes; the
 //    online softmax runs in base 2 per (lane, query head of the kv head's group).  Each K/V row
 //    is fetched once and reused from registers by every query head of its GQA group.
@@ -41,6 +47,8 @@
 //    64 page ids, so a workgroup starts its first K/V loads one round trip after launch instead
 //    of three (lengths -> offsets -> page ids -> rows).
 #pragma once
+
+#include <type_traits>
 
 #include "ifn_common.hpp"
 
@@ -63,7 +71,10 @@ constexpr int kRowStartCost = 24;
 // The cost the split charges a call's rows: none for a single row (every range then holds one
 // piece of it, so no range starts a second row), which keeps one row of 512 keys at 16 ranges
 // of 32 keys -- one burst per wave and one round trip of split states in the final merge.
-__host__ __device__ __forceinline__ int row_start_cost(int batch) { return batch > 1 ? kRowStartCost : 0; }
+// tpw: token rows a wave holds at once; the cost is a time, so it counts that many times the tokens
+// (planned, us: 4 kv heads, 48 rows of 100-4000 keys 46.7 with 24, 43.8 with 48; 2 kv heads, 32 such rows
+// 27.3 with 24, 23.1 with 96; equal rows lose a little: 64 rows of 3000, 4 kv heads, 67.4 and 69.1).
+__host__ __device__ __forceinline__ int row_start_cost(int batch, int tpw = 1) { return batch > 1 ? kRowStartCost * tpw : 0; }
 // Fewest virtual positions per range.  A row split over n ranges is merged by one workgroup that
 // reads n partial states (Hq x D floats each), so short batches are split over fewer workgroups:
 // one row of 512 keys takes 16 ranges of 32 positions instead of one range per CU.
@@ -82,9 +93,12 @@ __device__ __forceinline__ int64_t div_floor(int64_t num, int64_t den) {
 __device__ __forceinline__ int64_t range_count(int64_t nb, int64_t T) {
   return min(nb, (T + kMinRangePositions - 1) / kMinRangePositions);
 }
+// The step plan's last header word: the shared-prefix keys, or (smaller token rows, which have no shared
+// prefix) the rows a wave holds, negated -- their splits differ.
+__host__ __device__ __forceinline__ int plan_mode(int pk, int tpw) { return tpw > 1 ? -tpw : pk; }
 
 // Step plan (int32 words).  Header: magic, batch, ranges nr, virtual positions T, grid, whether
-// appended slots were given, the row-length cap, the shared-prefix keys pk (0: none).  Then the
+// appended slots were given, the row-length cap, plan_mode (the shared-prefix keys, 0: none).  Then the
 // rows' offsets cum[batch + 1], then one record per workgroup range: [0] pieces of the range;
 // [1 + 6 p ..] piece p < kPlanPieces: row, first key a, end key e, first range of the row, ranges of
 // the row, and the row's appended slot (or, in shared-prefix mode, which has no append, the key of
@@ -101,17 +115,18 @@ static inline size_t plan_words(int32_t batch, int blocks) { return size_t(plan_
 
 // Workspace: [tickets: kTicketBytes][ml][o].  Slot = row + range index: the workgroups holding a
 // row are consecutive ranges, so (row, range) -> row + range is unique and below batch + ranges.
-// A split state is (m, l) in fp32 and the normalised output O / l in fp16 (a convex combination of
-// value rows, so fp16 keeps it to a relative 2^-11): the last arrival of a long row reads every
-// state of it, and halving the bytes it reads halves that step.
+// A split state is (m, l) in fp32 and the normalised output O / l, in fp16 for 2 KiB token rows (a
+// convex combination of value rows, so fp16 keeps it to a relative 2^-11): the last arrival of a
+// long row reads every state of it, and halving the bytes it reads halves that step.  Smaller token
+// rows (f32) keep O / l in fp32.
 static inline size_t rows_ws_layout(int32_t batch, int32_t hq, int32_t d, int64_t ranges, size_t* off_ml,
-                                    size_t* off_o) {
+                                    size_t* off_o, bool f32 = false) {
   const size_t slots = size_t(batch) + size_t(ranges);
   size_t off = kTicketBytes;
   *off_ml = off;
   off = align256(off + slots * hq * 2 * sizeof(float));
   *off_o = off;
-  off = align256(off + slots * hq * d * sizeof(uint16_t));
+  off = align256(off + slots * hq * d * (f32 ? sizeof(float) : sizeof(uint16_t)));
   return off;
 }
 
@@ -136,7 +151,7 @@ __device__ __forceinline__ int row_slot(const int32_t* slots, const uint8_t* act
 // s_len (optional): the rows' keys, already in LDS (and published by a barrier).
 __device__ __forceinline__ int build_offsets(int* s_cum, int* s_wsum, const int32_t* seq_lens,
                                              const uint8_t* active, int batch, int cap, int pk = 0,
-                                             uint8_t* s_casc = nullptr, const int* s_len = nullptr) {
+                                             uint8_t* s_casc = nullptr, const int* s_len = nullptr, int tpw = 1) {
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave, nwaves = blockDim.x / kWave;
   int running = 0;
   for (int base = 0; base < batch; base += blockDim.x) {
@@ -145,7 +160,7 @@ __device__ __forceinline__ int build_offsets(int* s_cum, int* s_wsum, const int3
     const bool casc = pk > 0 && len >= pk;
     if (s_casc != nullptr && i < batch) s_casc[i] = casc ? 1 : 0;
     if (casc) len -= pk;
-    if (len > 0) len += row_start_cost(batch);
+    if (len > 0) len += row_start_cost(batch, tpw);
     int x = len;
 #pragma unroll
     for (int o = 1; o < kWave; o <<= 1) {
@@ -194,7 +209,7 @@ template <int PB>  // tokens per page
 __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(
     int32_t* __restrict__ plan, const int32_t* __restrict__ block_tables, int32_t max_pages,
     const int32_t* __restrict__ seq_lens, const uint8_t* __restrict__ active, const int32_t* __restrict__ slots,
-    int64_t num_pages, int32_t batch, int32_t max_len, int32_t nb, int32_t pk) {
+    int64_t num_pages, int32_t batch, int32_t max_len, int32_t nb, int32_t pk, int32_t tpw) {
   __shared__ int s_cum[kRowsMaxBatch + 1];
   __shared__ int s_wsum[kPlanThreads / kWave];
   __shared__ int s_p0[3][kPlanThreads];  // first piece of range r: row, a, e (rows < 0: none)
@@ -246,7 +261,7 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(
   }
   __syncthreads();
   // (pk > 0: a row of at least pk keys streams only its keys after the first pk)
-  const int T = build_offsets(s_cum, s_wsum, seq_lens, active, batch, cap, pk, nullptr, s_len);
+  const int T = build_offsets(s_cum, s_wsum, seq_lens, active, batch, cap, pk, nullptr, s_len, tpw);
   const int nr = int(range_count(nb, T));
   if (tid == 0) {
     plan[0] = kPlanMagic;
@@ -256,7 +271,7 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(
     plan[4] = nb;
     plan[5] = slots != nullptr ? 1 : 0;
     plan[6] = cap;
-    plan[7] = pk;
+    plan[7] = plan_mode(pk, tpw);
   }
   // (every word of the plan is written, so that a buffer needs no clearing and two plans compare equal)
   if (tid >= 8 && tid < kPlanHdr) plan[tid] = 0;
@@ -272,7 +287,7 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(
       auto range_of = [&](int64_t t) -> int { return int(div_floor((t + 1) * nr - 1, T)); };
       int b = locate_row(s_cum, batch, t0);
       while (b < batch) {
-        const int cb = s_cum[b] + row_start_cost(batch);
+        const int cb = s_cum[b] + row_start_cost(batch, tpw);
         const int len = s_cum[b + 1] - cb;
         if (len > 0) {
           if (cb >= t1) break;
@@ -383,11 +398,13 @@ __device__ __forceinline__ u32x4 pack_h8(const float (&x)[8]) {
 template <int D, int G, int HKV, bool kPrep, bool kCascade, int NT = 2>
 struct RowsLds {
   static constexpr int HQ = HKV * G, GR = G < 2 ? G : 2, ROW = HKV * D;
+  static constexpr int TPW = 2 * kWave * 8 / ROW;  // token rows a wave holds at once
+  static constexpr int VW = kRowsWaves * TPW;      // states per piece: one per token row in flight
   int (&s_cum)[kRowsMaxBatch + 1];  // rows' offsets in the virtual token list
   int (&s_wsum)[kRowsWaves];
-  float (&s_m)[kRowsWaves][HQ];
-  float (&s_l)[kRowsWaves][HQ];
-  f32x4 (&s_acc)[kRowsWaves][HKV * GR][D / 4];
+  float (&s_m)[VW][HQ];
+  float (&s_l)[VW][HQ];
+  f32x4 (&s_acc)[VW][HKV * GR][D / 4];
   uint32_t (&s_ticket)[NT];  // tickets taken at the end of a range (kFused: per kv head of two rows)
   uint8_t (&s_casc)[kCascade ? kRowsMaxBatch : 1];  // kCascade: row b is a cascade row
   // kPrep: the appended token's fp16 K and V rows, prepared at the start of its piece
@@ -396,17 +413,18 @@ struct RowsLds {
   f16 (&s_q)[kPrep ? G : 1][kPrep ? ROW : 8];
 };
 
-// The merges of the whole-row kernel, over split states (m, l) fp32 and O / l fp16 at slots of the
+// The merges of the whole-row kernel, over split states (m, l) fp32 and O / l fp16 (F32: fp32) at slots of the
 // workspace (r_ml, r_o) and, for a cascade row, its prefix states (px).  kDev: the prefix states were
 // written in the same launch, by other workgroups, so they are read at the device coherence point.
 // MB: split states per round trip.
-template <int D, int G, int HKV, bool kDev, int MB = kMergeBatch>
+template <int D, int G, int HKV, bool kDev, int MB = kMergeBatch, bool F32 = false>
 struct RowsMerge {
   static constexpr int HQ = HKV * G, D4 = D / 4;
   // A batch of split states (MB per round trip) and of prefix states (4 per round trip).
+  using State = std::conditional_t<F32, f32x4, f32x2>;  // 4 dims of O / l
   struct Ld {
     f32x2 ml[MB];
-    f32x2 o[MB];  // 4 fp16 dims of O / l
+    State o[MB];
   };
   struct Px {
     f32x2 ml[4];
@@ -418,7 +436,12 @@ struct RowsMerge {
 
   __device__ __forceinline__ uint32_t ml_off(int64_t s, int qh) const { return uint32_t((s * HQ + qh) * 2 * 4); }
   __device__ __forceinline__ uint32_t o_off(int64_t s, int qh, int d4) const {
-    return uint32_t(((s * HQ + qh) * D + 4 * d4) * 2);
+    return uint32_t(((s * HQ + qh) * D + 4 * d4) * (F32 ? 4 : 2));
+  }
+  // A state's 4 dims, O (normalised) to slot s.
+  __device__ __forceinline__ void put(int64_t s, int qh, int d4, f32x4 o) const {
+    if constexpr (F32) st_dev4(r_o, o_off(s, qh, d4), o);
+    else st_dev2(r_o, o_off(s, qh, d4), __builtin_bit_cast(f32x2, f16x4{f16(o[0]), f16(o[1]), f16(o[2]), f16(o[3])}));
   }
   // Log-sum-exp merge of a split row's np states (slots slot0 .. slot0 + np - 1, in range order)
   // for query head qh, dims 4 d4 .. 4 d4 + 3.  Every lane loads each state's (m, l) itself (the
@@ -432,7 +455,8 @@ struct RowsMerge {
     for (int u = 0; u < MB; ++u) {
       if (u < cnt) {
         ld.ml[u] = ld_dev2(r_ml, ml_off(s0 + u, qh));
-        ld.o[u] = ld_dev2(r_o, o_off(s0 + u, qh, d4));
+        if constexpr (F32) ld.o[u] = ld_dev4(r_o, o_off(s0 + u, qh, d4));
+        else ld.o[u] = ld_dev2(r_o, o_off(s0 + u, qh, d4));
       }
     }
   }
@@ -458,10 +482,15 @@ struct RowsMerge {
       for (int u = 0; u < MB; ++u) {
         if (u < cnt) {
           const float w = exp2_fast(ld.ml[u][0] - M) * ld.ml[u][1];  // weight of O / l: e^(m - M) l
-          const f16x4 oh = __builtin_bit_cast(f16x4, ld.o[u]);
+          f32x4 oh;
+          if constexpr (F32) {
+            oh = ld.o[u];
+          } else {
+            const f16x4 h = __builtin_bit_cast(f16x4, ld.o[u]);
+            oh = f32x4{float(h[0]), float(h[1]), float(h[2]), float(h[3])};
+          }
           L += w;
-          O = f32x4{fmaf(w, float(oh[0]), O[0]), fmaf(w, float(oh[1]), O[1]), fmaf(w, float(oh[2]), O[2]),
-                    fmaf(w, float(oh[3]), O[3])};
+          O = f32x4{fmaf(w, oh[0], O[0]), fmaf(w, oh[1], O[1]), fmaf(w, oh[2], O[2]), fmaf(w, oh[3], O[3])};
         }
       }
     }
@@ -565,13 +594,17 @@ __device__ __forceinline__ void decode_rows_body(
     const int32_t* block_tables, const f16* q, int32_t batch, int32_t max_pages, int32_t max_len, int32_t nb_arg,
     int64_t num_pages, f16* out, const int32_t* seq_lens, const uint8_t* active, float scale_log2, DecodeWorkspace ws,
     DecodeAppend ap, DecodePrep pp, DecodePrefix px) {
-  constexpr int LPH = kWave / HKV;  // lanes per kv head
   constexpr int ROW = HKV * D;      // fp16 elements per token row
+  constexpr int TPW = 2 * kWave * 8 / ROW;   // token rows per wave and load
+  constexpr int LPT = kWave / TPW;  // lanes per token row
+  constexpr int LPH = LPT / HKV;    // lanes per kv head
+  constexpr int VW = kRowsWaves * TPW;
   constexpr int HQ = HKV * G;
   constexpr int GR = G < 2 ? G : 2;  // query heads per kv head merged per LDS round
   constexpr int D4 = D / 4;
   constexpr bool kApp = kAppend || kPrep;  // the step's appended rows are stored by this launch
-  static_assert(ROW == 2 * kWave * 8, "a token row is two 16-byte chunks per lane");
+  static_assert(TPW * ROW == 2 * kWave * 8 && TPW <= PB, "whole token rows, two 16-byte chunks per lane");
+  static_assert(TPW == 1 || (!kPrep && !kCascade), "one token row per wave in these modes");
   static_assert(G % GR == 0, "merge rounds cover the group");
   static_assert(!(kAppend && kPrep), "one append mode");
   static_assert(!(kCascade && (kAppend || kPrep)), "shared-prefix mode has no append");
@@ -598,11 +631,12 @@ __device__ __forceinline__ void decode_rows_body(
   const int64_t blk = (nbi % kRowsXcds) == 0 ? (bid % kRowsXcds) * (nbi / kRowsXcds) + bid / kRowsXcds : bid;
   // split partials: O [slot][HQ][D] and (m, l) [slot][HQ][2], slot < batch + grid; and the merges
   const uint32_t n_slots = uint32_t(batch) + uint32_t(nb);
-  const __amdgpu_buffer_rsrc_t r_o = make_rsrc(ws.o, n_slots * HQ * D * 2u);
+  constexpr bool kF32 = TPW > 1;  // split states' O / l
+  const __amdgpu_buffer_rsrc_t r_o = make_rsrc(ws.o, n_slots * HQ * D * (kF32 ? 4u : 2u));
   const __amdgpu_buffer_rsrc_t r_ml = make_rsrc(ws.ml, n_slots * HQ * 2u * 4u);
   // (kFused: 4 split states per round trip -- a cascade row's private keys span few ranges -- which
   // keeps the merges' scalar registers few in a kernel that shares them with the prefix pass)
-  using MG = RowsMerge<D, G, HKV, kFused, kFused ? kFusedMergeBatch : kMergeBatch>;
+  using MG = RowsMerge<D, G, HKV, kFused, kFused ? kFusedMergeBatch : kF32 ? kMergeBatch / 2 : kMergeBatch, kF32>;
   using PxBatch = typename MG::Px;
   using MergeLd = typename MG::Ld;
   const MG mg{r_o, r_ml, px, out};
@@ -627,7 +661,7 @@ __device__ __forceinline__ void decode_rows_body(
     ids_pl = rec[64 + lane];
     cum_pf = plan[kPlanHdr + min(tid, batch)];
     planned = (h0[0] == kPlanMagic) & (h0[1] == batch) & (h1[0] == int(nb)) & (h1[2] == cap) &
-              (!kApp | (h1[1] != 0)) & (h1[3] == pk);
+              (!kApp | (h1[1] != 0)) & (h1[3] == plan_mode(pk, TPW));
     T = h0[3];
     rec_n = rec_a[0];
   }
@@ -750,7 +784,7 @@ __device__ __forceinline__ void decode_rows_body(
 
   // Unplanned (or a plan for other shapes): the offsets are built here, before anything else.
   // Planned: they go to LDS at the first merge barrier, for pieces the record does not describe.
-  if (!planned) T = build_offsets(s_cum, s_wsum, seq_lens, active, batch, cap, pk, kCascade ? s_casc : nullptr);
+  if (!planned) T = build_offsets(s_cum, s_wsum, seq_lens, active, batch, cap, pk, kCascade ? s_casc : nullptr, nullptr, TPW);
   bool have_cum = !planned;
   // ws.plan_out (an unplanned call that builds the step's plan for the later layers): the same words
   // decode_plan_kernel writes -- workgroup 0 the header and the offsets, each workgroup its range's
@@ -766,7 +800,7 @@ __device__ __forceinline__ void decode_rows_body(
       pout[4] = int(nb);
       pout[5] = kApp ? 1 : 0;
       pout[6] = cap;
-      pout[7] = pk;
+      pout[7] = plan_mode(pk, TPW);
     }
     if (tid >= 8 && tid < kPlanHdr) pout[tid] = 0;
     for (int i = kPlanHdr + tid; i < plan_rec0(batch); i += kRowsThreads)
@@ -798,7 +832,7 @@ __device__ __forceinline__ void decode_rows_body(
     P.nranges = 1;
     int b = prev < 0 ? locate_row(s_cum, batch, t0) : prev + 1;
     for (; b < batch; ++b) {
-      const int cb = s_cum[b] + row_start_cost(batch);
+      const int cb = s_cum[b] + row_start_cost(batch, TPW);
       const int len = s_cum[b + 1] - cb;
       if (len <= 0) continue;
       if (cb >= t1) break;
@@ -841,7 +875,8 @@ __device__ __forceinline__ void decode_rows_body(
     return P;
   };
 
-  const int hd = lane / LPH, col = lane % LPH;
+  const int sub = lane / LPT;  // which of the wave's token rows
+  const int hd = lane % LPT / LPH, col = lane % LPH;
   const int off0 = hd * D + 8 * col, off1 = off0 + 8 * LPH;  // this lane's two chunks of a token row
   const int64_t v_off = num_pages * PB * int64_t(ROW);
 
@@ -941,12 +976,12 @@ __device__ __forceinline__ void decode_rows_body(
     if (prec != nullptr && pi == 0 && wave == 0) prec[kPlanIds + lane] = ids0;  // the first window's page ids
     int cur_w = 0;
 
-    // this wave's tokens: positions a + wave + 8 i, i < nw
-    const int rem = e - a - wave;
+    // this wave's tokens: positions a + (wave + 8 i) TPW + 0 .. TPW - 1, i < nw
+    const int rem = TPW == 1 ? e - a - wave : (e - a + TPW - 1) / TPW - wave;
     const int nw = rem > 0 ? (rem + kRowsWaves - 1) / kRowsWaves : 0;
-    auto rel_page = [&](int i) { return (a + wave + kRowsWaves * i) / PB - pg0; };
-    auto page_of = [&](int i) -> int {
-      const int rp = rel_page(i);
+    auto first_pos = [&](int i) { return a + wave * TPW + kRowsWaves * TPW * i; };
+    auto rel_page = [&](int i) { return first_pos(i) / PB - pg0; };
+    auto page_at = [&](int rp) -> int {
       return (rp >> 6) == cur_w ? __builtin_amdgcn_readlane(ids0, rp & 63) : __builtin_amdgcn_readlane(ids1, rp & 63);
     };
     auto shift = [&](int i) {  // token i's page enters the next 64-page window of the piece
@@ -956,9 +991,17 @@ __device__ __forceinline__ void decode_rows_body(
         ids1 = bt[min(kWave * (cur_w + 1) + lane, npg - 1)];
       }
     };
+    // (ok: the token is in the piece and its page in the pool; uniform when TPW == 1)
     auto issue = [&](int i, u32x4 (&kr)[2], u32x4 (&vr)[2], bool& ok) {
-      const int p = a + wave + kRowsWaves * i;
-      const int phys = page_of(i);
+      int p = first_pos(i), phys = page_at(p / PB - pg0);
+      bool in = true;
+      if constexpr (TPW > 1) {  // a wave's rows lie on at most two pages
+        const int p1 = min(p + TPW - 1, e - 1), rp0 = p / PB;
+        const int phys1 = page_at(p1 / PB - pg0);
+        in = p + sub < e;
+        p = min(p + sub, e - 1);
+        phys = p / PB == rp0 ? phys : phys1;
+      }
       ok = phys >= 0 && int64_t(phys) < num_pages;
       const int64_t tok = int64_t(ok ? phys : 0) * PB + p % PB;
       const f16* kb = pool + tok * ROW;
@@ -969,6 +1012,7 @@ __device__ __forceinline__ void decode_rows_body(
           vb = ap.new_v + int64_t(b) * ROW;
         }
       }
+      ok = ok && in;
       kr[0] = kStream ? ld16_stream(kb + off0) : ld16(kb + off0);
       kr[1] = kStream ? ld16_stream(kb + off1) : ld16(kb + off1);
       vr[0] = kStream ? ld16_stream(vb + off0) : ld16(vb + off0);
@@ -984,9 +1028,15 @@ __device__ __forceinline__ void decode_rows_body(
       for (int j = 0; j < 16; ++j) acc[g][j] = 0.f;
     }
     auto consume = [&](u32x4 (&kr)[2], u32x4 (&vr)[2], bool ok) {
-      if (!ok) {  // a page id outside the pool contributes no key (uniform)
-        vr[0] = u32x4{0u, 0u, 0u, 0u};
-        vr[1] = u32x4{0u, 0u, 0u, 0u};
+      // (a page id outside the pool contributes no key; both branches are uniform)
+      if constexpr (TPW == 1) {
+        if (!ok) {
+          vr[0] = u32x4{0u, 0u, 0u, 0u};
+          vr[1] = u32x4{0u, 0u, 0u, 0u};
+        }
+      } else if (__builtin_amdgcn_ballot_w64(!ok) != 0) {
+        vr[0] = ok ? vr[0] : u32x4{0u, 0u, 0u, 0u};
+        vr[1] = ok ? vr[1] : u32x4{0u, 0u, 0u, 0u};
       }
       float vf[16];
       const f16x8 v0 = as_h8(vr[0]), v1 = as_h8(vr[1]);
@@ -1106,8 +1156,8 @@ __device__ __forceinline__ void decode_rows_body(
     if (col == 0) {
 #pragma unroll
       for (int g = 0; g < G; ++g) {
-        s_m[wave][hd * G + g] = m[g];
-        s_l[wave][hd * G + g] = l[g];
+        s_m[wave * TPW + sub][hd * G + g] = m[g];
+        s_l[wave * TPW + sub][hd * G + g] = l[g];
       }
     }
 #pragma unroll
@@ -1115,7 +1165,7 @@ __device__ __forceinline__ void decode_rows_body(
 #pragma unroll
       for (int gg = 0; gg < GR; ++gg) {
         const int g = r * GR + gg;
-        f32x4* dst = s_acc[wave][hd * GR + gg];
+        f32x4* dst = s_acc[wave * TPW + sub][hd * GR + gg];
         dst[2 * col] = f32x4{acc[g][0], acc[g][1], acc[g][2], acc[g][3]};
         dst[2 * col + 1] = f32x4{acc[g][4], acc[g][5], acc[g][6], acc[g][7]};
         dst[2 * (col + LPH)] = f32x4{acc[g][8], acc[g][9], acc[g][10], acc[g][11]};
@@ -1127,17 +1177,17 @@ __device__ __forceinline__ void decode_rows_body(
         const int qh = item_qh(r);
         PxBatch pb;
         if (kCascade && !publish && P.off > 0) mg.px_load(b, qh, d4, 0, pb);
-        float mw[kRowsWaves];
+        float mw[VW];
         float M = kNegBig;
 #pragma unroll
-        for (int w = 0; w < kRowsWaves; ++w) {
+        for (int w = 0; w < VW; ++w) {
           mw[w] = s_m[w][qh];
           M = fmaxf(M, mw[w]);
         }
         float L = 0.f;
         f32x4 O = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int w = 0; w < kRowsWaves; ++w) {
+        for (int w = 0; w < VW; ++w) {
           const float wt = exp2_fast(mw[w] - M);
           L = fmaf(wt, s_l[w][qh], L);
           const f32x4 a4 = s_acc[w][hg][d4];
@@ -1147,8 +1197,7 @@ __device__ __forceinline__ void decode_rows_body(
           mg.write_row(b, qh, d4, M, L, O, kCascade && P.off > 0, pb);
         } else {  // publish this range's state of the row; its ticket is taken at the end
           const float inv = L > 0.f ? 1.f / L : 0.f;
-          const f16x4 oh = f16x4{f16(O[0] * inv), f16(O[1] * inv), f16(O[2] * inv), f16(O[3] * inv)};
-          st_dev2(r_o, mg.o_off(slot, qh, d4), __builtin_bit_cast(f32x2, oh));
+          mg.put(slot, qh, d4, f32x4{O[0] * inv, O[1] * inv, O[2] * inv, O[3] * inv});
           if (d4 == 0) st_dev2(r_ml, mg.ml_off(slot, qh), f32x2{M, L});
         }
       }
@@ -1311,9 +1360,9 @@ __global__ __launch_bounds__(kRowsThreads) void decode_rows_kernel(
   using L = RowsLds<D, G, HKV, kPrep, kCascade>;
   __shared__ int s_cum[kRowsMaxBatch + 1];
   __shared__ int s_wsum[kRowsWaves];
-  __shared__ float s_m[kRowsWaves][L::HQ];
-  __shared__ float s_l[kRowsWaves][L::HQ];
-  __shared__ f32x4 s_acc[kRowsWaves][HKV * L::GR][D / 4];
+  __shared__ float s_m[L::VW][L::HQ];
+  __shared__ float s_l[L::VW][L::HQ];
+  __shared__ f32x4 s_acc[L::VW][HKV * L::GR][D / 4];
   __shared__ uint32_t s_ticket[2];
   __shared__ uint8_t s_casc[kCascade ? kRowsMaxBatch : 1];
   __shared__ __attribute__((aligned(16))) f16 s_app[kPrep ? 2 : 1][kPrep ? L::ROW : 8];

@@ -740,11 +740,18 @@ extern "C" size_t ifn_paged_decode_workspace_bytes(int32_t batch, int32_t num_q_
   const int blocks = ifn::decode_blocks();
   const size_t per_head = ifn::decode_ws_layout(batch, num_kv_heads, num_q_heads / num_kv_heads, head_dim,
                                                 int64_t(blocks) * ifn::kWavesPerBlock, &off_ml, &off_o);
-  const size_t rows = ifn::rows_decode_ws_bytes(batch, num_q_heads, head_dim, blocks);
+  const size_t rows = ifn::rows_decode_ws_bytes(batch, num_q_heads, num_kv_heads, head_dim, blocks);
   return per_head > rows ? per_head : rows;
 }
 
 namespace ifn {
+
+// Whether a call's plan buffer is an error when it cannot hold a plan (2 KiB token rows).
+static bool plan_required(int32_t hkv, int32_t d) { return hkv * d >= 1024; }
+static bool plan_usable(const void* plan, size_t plan_bytes, int32_t batch) {
+  return plan != nullptr && (reinterpret_cast<uintptr_t>(plan) & 15u) == 0 &&
+         plan_bytes >= rows_plan_bytes(std::max(batch, 1), decode_blocks());
+}
 
 // ifn_paged_decode, ifn_paged_decode_append and ifn_paged_decode_shared_prefix with no shared
 // pages: the same checks and launch; `ap` carries the fused append (kAppend variant) when its
@@ -778,8 +785,12 @@ static int decode_entry(void* out, const void* query, const void* kv_pool_layer,
   if (!rows && k == nullptr) return IFN_ERR_UNSUPPORTED;
   if (prep != nullptr && (!rows || !rows_prep_supported(num_q_heads, num_kv_heads, head_dim)))
     return IFN_ERR_UNSUPPORTED;
-  // (a call that builds the step's plan needs somewhere to write it, where the shape has a plan)
-  if (build_plan && rows && batch > 0 && plan == nullptr) return IFN_ERR_INVALID_ARGUMENT;
+  // (a call that builds the step's plan needs somewhere to write it, where the shape has a plan.  Token
+  // rows below 2 KiB had none when their callers were written: there a missing or unusable plan buffer
+  // means no plan)
+  const bool whole = plan_required(num_kv_heads, head_dim);
+  if (!whole && !plan_usable(plan, plan_bytes, batch)) plan = nullptr;
+  if (build_plan && rows && whole && batch > 0 && plan == nullptr) return IFN_ERR_INVALID_ARGUMENT;
   IFN_CHECK_ALIGN16(out);
   IFN_CHECK_ALIGN16(query);
   IFN_CHECK_ALIGN16(kv_pool_layer);
@@ -882,12 +893,14 @@ extern "C" int ifn_paged_decode_plan(void* plan, size_t plan_bytes, const int32_
   if (batch == 0) return IFN_OK;
   if (!rows_decode_supported(batch, num_q_heads, num_kv_heads, head_dim, max_pages_per_seq, max_seq_len, block_size))
     return block_size == kBlock ? IFN_OK : IFN_ERR_UNSUPPORTED;  // 16: these shapes decode without a plan
+  if (!plan_required(num_kv_heads, head_dim) && !plan_usable(plan, plan_bytes, batch)) return IFN_OK;
   const int blocks = decode_blocks();
   if (plan == nullptr || plan_bytes < rows_plan_bytes(batch, blocks)) return IFN_ERR_WORKSPACE;
   IFN_CHECK_ALIGN16(plan);
   if (device_cu_count() < 1) return IFN_ERR_HIP;
   return rows_plan_launch(static_cast<int32_t*>(plan), block_tables, max_pages_per_seq, seq_lens, active_mask,
-                          slot_mapping, num_pages, batch, max_seq_len, blocks, reinterpret_cast<hipStream_t>(stream),
+                          slot_mapping, num_pages, batch, max_seq_len, blocks, num_kv_heads, head_dim,
+                          reinterpret_cast<hipStream_t>(stream),
                           block_size);
 }
 
@@ -1031,7 +1044,7 @@ static SharedLayout shared_layout(int32_t batch, int32_t hkv, int32_t g, int32_t
   SharedLayout L;
   size_t off_ml, off_o;
   const size_t dec = std::max(decode_ws_layout(batch, hkv, g, d, waves, &off_ml, &off_o),
-                              rows_decode_ws_bytes(batch, hkv * g, d, int(waves / kWavesPerBlock)));
+                              rows_decode_ws_bytes(batch, hkv * g, hkv, d, int(waves / kWavesPerBlock)));
   L.nstates = prefix_pass_splits(batch, hkv * g, hkv, d, key_len, cus) + 1;  // <= kMaxStates
   const size_t states = size_t(batch) * hkv * L.nstates * g;
   L.dec_ml = off_ml;
@@ -1057,7 +1070,7 @@ extern "C" size_t ifn_paged_decode_shared_prefix_workspace_bytes(int32_t batch, 
                                            int64_t(blocks) * ifn::kWavesPerBlock, shared_pages * block_size, cus)
                             .bytes;
   // shared_pages == 0 runs the plain decode (whole-row kernel where compiled)
-  const size_t rows = ifn::rows_decode_ws_bytes(batch, num_q_heads, head_dim, blocks);
+  const size_t rows = ifn::rows_decode_ws_bytes(batch, num_q_heads, num_kv_heads, head_dim, blocks);
   return shared > rows ? shared : rows;
 }
 
@@ -1085,7 +1098,8 @@ static int shared_prefix_entry(void* out, const void* query, const void* kv_pool
   if (batch > kMaxBatch || int64_t(batch) * num_kv_heads > kMaxTickets) return IFN_ERR_UNSUPPORTED;
   const int g = num_q_heads / num_kv_heads;
   // the private pages on the whole-row kernel where it compiles the shape, else per segment
-  const bool rows = rows_decode_supported(batch, num_q_heads, num_kv_heads, head_dim, max_pages_per_seq, max_seq_len);
+  const bool rows = rows_decode_supported(batch, num_q_heads, num_kv_heads, head_dim, max_pages_per_seq, max_seq_len) &&
+                    rows_cascade_supported(num_q_heads, num_kv_heads, head_dim);
   DecodeKernel k = rows ? nullptr : pick_decode(head_dim, g, DecodeMode::kCascade);
   CombineKernel kc = pick_combine(head_dim);
   if ((!rows && k == nullptr) || kc == nullptr) return IFN_ERR_UNSUPPORTED;
@@ -1201,11 +1215,14 @@ extern "C" int ifn_paged_decode_shared_prefix_plan(void* plan, size_t plan_bytes
   if (block_size != kBlock) return IFN_ERR_UNSUPPORTED;
   if (!rows_decode_supported(batch, num_q_heads, num_kv_heads, head_dim, max_pages_per_seq, max_seq_len, block_size))
     return IFN_OK;  // these shapes decode without a plan
+  if (!plan_required(num_kv_heads, head_dim) &&
+      (shared_pages > 0 || !plan_usable(plan, plan_bytes, batch)))  // (the shared-prefix form takes none)
+    return IFN_OK;
   const int blocks = decode_blocks();
   if (plan == nullptr || plan_bytes < rows_plan_bytes(batch, blocks)) return IFN_ERR_WORKSPACE;
   IFN_CHECK_ALIGN16(plan);
   if (device_cu_count() < 1) return IFN_ERR_HIP;
   return rows_plan_launch(static_cast<int32_t*>(plan), block_tables, max_pages_per_seq, seq_lens, active_mask, nullptr,
-                          num_pages, batch, max_seq_len, blocks, reinterpret_cast<hipStream_t>(stream), block_size,
-                          shared_pages * block_size);
+                          num_pages, batch, max_seq_len, blocks, num_kv_heads, head_dim, reinterpret_cast<hipStream_t>(stream),
+                          block_size, shared_pages * block_size);
 }

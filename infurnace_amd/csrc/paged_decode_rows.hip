@@ -25,6 +25,16 @@ static RowsKernel pick_rows(int d, int g, int hkv, bool append, bool stream, boo
     return stream ? decode_rows_kernel<DD, GG, HH, kRowsStages, false, true>                       \
                   : decode_rows_kernel<DD, GG, HH, kRowsStages, false, false>;                     \
   }
+  // Token rows of 1 KiB and 512 B (tensor-parallel shards of the Qwen3 shapes over 2 and 4 GPUs, 8 x 64):
+  // plain and fused-append variants; faster than the per-head kernel at every size measured
+  // (decode_rows.hpp).
+#define IFN_ROWS_SHARD(DD, GG, HH)                                                                 \
+  if (d == DD && g == GG && hkv == HH) {                                                           \
+    if (prep || cascade) return nullptr;                                                           \
+    if (append) return decode_rows_kernel<DD, GG, HH, kRowsStages, true, true>;                    \
+    return stream ? decode_rows_kernel<DD, GG, HH, kRowsStages, false, true>                       \
+                  : decode_rows_kernel<DD, GG, HH, kRowsStages, false, false>;                     \
+  }
   // Pages of 32 and 64 tokens (the page-size choice is benchmarked on them): Qwen3 decode shapes,
   // plain (streaming or cached loads) and fused-append variants.
 #define IFN_ROWS_PAGES(DD, GG, HH, PP)                                                                           \
@@ -38,43 +48,53 @@ static RowsKernel pick_rows(int d, int g, int hkv, bool append, bool stream, boo
     IFN_ROWS_CASE(128, 1, 8) IFN_ROWS_CASE(128, 2, 8) IFN_ROWS_CASE(128, 4, 8)
     IFN_ROWS_CASE(64, 1, 16) IFN_ROWS_CASE(64, 2, 16)
     IFN_ROWS_CASE(256, 1, 4) IFN_ROWS_CASE(256, 2, 4)
+    IFN_ROWS_SHARD(128, 2, 4) IFN_ROWS_SHARD(128, 4, 4) IFN_ROWS_SHARD(128, 2, 2) IFN_ROWS_SHARD(128, 4, 2)
+    IFN_ROWS_SHARD(64, 2, 8)
   }
   IFN_ROWS_PAGES(128, 2, 8, 32) IFN_ROWS_PAGES(128, 4, 8, 32)
   IFN_ROWS_PAGES(128, 2, 8, 64) IFN_ROWS_PAGES(128, 4, 8, 64)
 #undef IFN_ROWS_PAGES
+#undef IFN_ROWS_SHARD
 #undef IFN_ROWS_CASE
   return nullptr;
 }
+
+// Token rows a wave holds at once.
+static int rows_per_wave(int32_t hkv, int32_t d) { return std::max(1, 1024 / std::max(1, hkv * d)); }
 
 bool rows_prep_supported(int32_t hq, int32_t hkv, int32_t d) {
   return hkv >= 1 && hq % hkv == 0 && pick_rows(d, hq / hkv, hkv, false, true, true) != nullptr;
 }
 
+bool rows_cascade_supported(int32_t hq, int32_t hkv, int32_t d) {
+  return hkv >= 1 && hq % hkv == 0 && pick_rows(d, hq / hkv, hkv, false, true, false, true) != nullptr;
+}
+
 bool rows_decode_supported(int32_t batch, int32_t hq, int32_t hkv, int32_t d, int32_t max_pages, int32_t max_len,
                            int32_t block_size, bool append) {
-  // the virtual token list must fit int32: batch * (cap + kRowStartCost) < 2^31
+  // the virtual token list must fit int32: batch * (cap + the row start cost) < 2^31
   const int64_t cap = std::min<int64_t>(int64_t(max_pages) * block_size, max_len);
   return batch >= 1 && batch <= kRowsMaxBatch && hq % hkv == 0 && batch <= kMaxTickets &&
-         int64_t(batch) * (cap + kRowStartCost) < (int64_t(1) << 31) &&
+         int64_t(batch) * (cap + kRowStartCost * rows_per_wave(hkv, d)) < (int64_t(1) << 31) &&
          pick_rows(d, hq / hkv, hkv, append, true, false, false, block_size) != nullptr;
 }
 
-size_t rows_decode_ws_bytes(int32_t batch, int32_t hq, int32_t d, int blocks) {
+size_t rows_decode_ws_bytes(int32_t batch, int32_t hq, int32_t hkv, int32_t d, int blocks) {
   size_t off_ml, off_o;
-  return rows_ws_layout(batch, hq, d, blocks, &off_ml, &off_o);
+  return rows_ws_layout(batch, hq, d, blocks, &off_ml, &off_o, hkv * d < 1024);
 }
 
 size_t rows_plan_bytes(int32_t batch, int blocks) { return plan_words(batch, blocks) * sizeof(int32_t); }
 
 int rows_plan_launch(int32_t* plan, const int32_t* block_tables, int32_t max_pages, const int32_t* seq_lens,
                      const uint8_t* active, const int32_t* slots, int64_t num_pages, int32_t batch, int32_t max_len,
-                     int blocks, hipStream_t stream, int32_t block_size, int32_t prefix_keys) {
+                     int blocks, int32_t hkv, int32_t d, hipStream_t stream, int32_t block_size, int32_t prefix_keys) {
   auto k = block_size == 64 ? decode_plan_kernel<64> : block_size == 32 ? decode_plan_kernel<32>
                                                                          : decode_plan_kernel<kRowsBlock>;
   if (block_size != kRowsBlock && block_size != 32 && block_size != 64) return IFN_ERR_UNSUPPORTED;
   if (prefix_keys < 0 || (prefix_keys > 0 && slots != nullptr)) return IFN_ERR_INVALID_ARGUMENT;
   k<<<dim3(1), dim3(kPlanThreads), 0, stream>>>(plan, block_tables, max_pages, seq_lens, active, slots, num_pages,
-                                                batch, max_len, blocks, prefix_keys);
+                                                batch, max_len, blocks, prefix_keys, rows_per_wave(hkv, d));
   return ifn_launch_status();
 }
 
@@ -87,7 +107,7 @@ int rows_decode_launch(f16* out, const f16* q, const f16* pool, int64_t num_page
   RowsKernel k = pick_rows(d, hq / hkv, hkv, ap.pool != nullptr, !cached, prep != nullptr, px != nullptr, block_size);
   if (k == nullptr) return IFN_ERR_UNSUPPORTED;
   size_t off_ml, off_o;
-  rows_ws_layout(batch, hq, d, blocks, &off_ml, &off_o);
+  rows_ws_layout(batch, hq, d, blocks, &off_ml, &off_o, hkv * d < 1024);
   uint8_t* wsb = static_cast<uint8_t*>(workspace);
   DecodeWorkspace ws;
   ws.count = reinterpret_cast<uint32_t*>(wsb);

@@ -165,8 +165,8 @@ def decode_plan(query_shape, kv_pool: torch.Tensor, block_tables: torch.Tensor, 
     nbytes = lib.ifn_paged_decode_plan_bytes(n, hq, hkv, d, bs, max_pages, msl)
     if nbytes == 0:
         return DecodePlan(None, 0, key)
-    # (the kernels write every word of a plan)
-    buf = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    # (the kernels write every word of a plan; a shared-prefix plan is left alone for some shapes)
+    buf = (torch.zeros if sp else torch.empty)(nbytes, dtype=torch.uint8, device=dev)
 
     def rebuild():
         return decode_plan(query_shape, kv_pool, block_tables, sequence_lengths, active_mask, slot_mapping,
