@@ -2,7 +2,8 @@
 
 ``python -m infurnace_amd.build`` compiles every ``csrc/*.hip`` with hipcc for
 gfx950 into ``_build/`` and links ``infurnace_amd/libinfurnace_hip.so`` in
-place (git-ignored; it travels to the GPU box with the source tree).
+place, beside ``_fast_call.so`` (the wrappers' native argument checks); both are
+git-ignored and travel to the GPU box with the source tree.
 
 Packed fp32 VALU forms are switched off for device code
 (``-target-feature -packed-fp32-ops``); hipcc's host pass warns that it does
@@ -15,12 +16,14 @@ import glob
 import os
 import subprocess
 import sys
+import sysconfig
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
 CSRC = os.path.join(PKG, "csrc")
 BUILD_DIR = os.path.join(ROOT, "_build")
 LIB_PATH = os.path.join(PKG, "libinfurnace_hip.so")
+FAST_PATH = os.path.join(PKG, "_fast_call.so")
 ARCH = "gfx950"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -68,6 +71,23 @@ def _compile(src: str) -> str:
     return obj
 
 
+def _build_fast() -> str:
+    """The wrappers' native argument checks (csrc/fast_call.cpp), a CPython extension against torch's headers."""
+    import torch
+    troot = os.path.dirname(torch.__file__)
+    tmp = FAST_PATH + ".tmp"
+    cmd = ["g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-isystem", f"{troot}/include",
+           "-isystem", sysconfig.get_paths()["include"], "-isystem", "/opt/rocm/include",
+           os.path.join(CSRC, "fast_call.cpp"), "-o", tmp, f"-L{troot}/lib", "-lc10", "-lc10_hip", "-ltorch_cpu",
+           "-ltorch_python"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed for fast_call.cpp:\n{r.stderr}")
+    os.replace(tmp, FAST_PATH)
+    return FAST_PATH
+
+
 def sources() -> list[str]:
     return sorted(glob.glob(os.path.join(CSRC, "*.hip")))
 
@@ -77,7 +97,9 @@ def build(jobs: int = 8) -> str:
     os.makedirs(BUILD_DIR, exist_ok=True)
     srcs = sources()
     with cf.ThreadPoolExecutor(max_workers=max(1, min(jobs, len(srcs)))) as ex:
+        fast = ex.submit(_build_fast)
         objs = list(ex.map(_compile, srcs))
+        fast.result()
     tmp = LIB_PATH + ".tmp"
     cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs]
     subprocess.run(cmd, check=True)

@@ -1,0 +1,58 @@
+"""Native forms of the wrappers' checks and calls (csrc/fast_call.cpp).
+
+Each function takes a wrapper's arguments in order, and either makes the call and returns its result or
+returns None with nothing launched: the arguments are then for the checked Python path, which
+accepts more forms (array carriers, host values) and raises the errors.  Without the extension every
+call takes that path.
+"""
+from __future__ import annotations
+
+import ctypes
+import importlib.util
+import os
+
+from .. import _capi
+
+EXT_PATH = os.path.join(os.path.dirname(_capi.LIB_PATH), "_fast_call.so")
+_NAMES = ("decode", "prep_decode", "prefill", "prep_prefill", "prep_append", "store", "store_layers")
+# the C entry points the extension calls, in the order it takes their addresses
+_ENTRIES = ("ifn_store_kv", "ifn_store_kv_layers", "ifn_paged_decode_workspace_bytes", "ifn_paged_decode",
+            "ifn_paged_decode_append", "ifn_paged_decode_planned", "ifn_paged_decode_append_planned",
+            "ifn_paged_decode_planning", "ifn_paged_decode_append_planning",
+            "ifn_paged_decode_shared_prefix_workspace_bytes", "ifn_paged_decode_shared_prefix",
+            "ifn_paged_prefill_workspace_bytes", "ifn_paged_prefill", "ifn_paged_prefill_append",
+            "ifn_qk_norm_rope_append", "ifn_paged_decode_prep_append", "ifn_paged_decode_prep_append_planning",
+            "ifn_paged_prefill_prep_append")
+
+
+def _none(*args):
+    return None
+
+
+def load():
+    """The extension, bound to the loaded library's entry points."""
+    lib = _capi.lib()
+    spec = importlib.util.spec_from_file_location("_fast_call", EXT_PATH)
+    ext = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(ext)
+    ext.bind(*(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in _ENTRIES))
+    return ext
+
+
+def _first(name):
+    def call(*args):
+        try:
+            _capi.lib()
+        except _capi.NativeLibraryError:
+            return None  # (the Python path says what is missing)
+        try:
+            ext = load()
+        except (ImportError, OSError):
+            ext = None
+        for n in _NAMES:
+            globals()[n] = _none if ext is None else getattr(ext, n)
+        return globals()[name](*args)
+    return call
+
+
+decode, prep_decode, prefill, prep_prefill, prep_append, store, store_layers = (_first(n) for n in _NAMES)

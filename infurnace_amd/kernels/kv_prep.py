@@ -22,6 +22,7 @@ import numpy as np
 import torch
 
 from .. import _capi
+from . import _fast
 from ._common import KVStoreError, PagedAttentionError, check_pool, current_stream, ptr
 from ._carrier import accepts_carriers
 
@@ -68,7 +69,6 @@ def _i32(name: str, t, n: int, device, dtypes=(torch.int32,)) -> torch.Tensor:
     return t
 
 
-@accepts_carriers
 def qk_norm_rope_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_norm_weight: torch.Tensor,
                         k_norm_weight: torch.Tensor, rope: torch.Tensor, positions: torch.Tensor,
                         slot_mapping: torch.Tensor, active_mask: torch.Tensor | None, kv_pool: torch.Tensor, *,
@@ -80,6 +80,19 @@ def qk_norm_rope_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_nor
     None.  A token whose position is outside the table stores nothing and gets a zero
     q row.
     """
+    o = _fast.prep_append(q, k, v, q_norm_weight, k_norm_weight, rope, positions, slot_mapping, active_mask, kv_pool,
+                          layer, eps, q_out)
+    if o is not None:
+        return o
+    return _qk_norm_rope_append(q, k, v, q_norm_weight, k_norm_weight, rope, positions, slot_mapping, active_mask,
+                                kv_pool, layer=layer, eps=eps, q_out=q_out)
+
+
+@accepts_carriers
+def _qk_norm_rope_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_norm_weight: torch.Tensor,
+                         k_norm_weight: torch.Tensor, rope: torch.Tensor, positions: torch.Tensor,
+                         slot_mapping: torch.Tensor, active_mask: torch.Tensor | None, kv_pool: torch.Tensor, *,
+                         layer: int = 0, eps: float = 1e-6, q_out: torch.Tensor | None = None) -> torch.Tensor:
     pool_layer, (P, bs, hkv, d) = check_pool(kv_pool, layer, KVStoreError)
     dev = pool_layer.device
     if not isinstance(q, torch.Tensor) or q.ndim != 3:
@@ -146,7 +159,6 @@ def copy_pages(kv_pool: torch.Tensor, src_ids: torch.Tensor, dst_ids: torch.Tens
                current_stream(kv_pool.device))
 
 
-@accepts_carriers
 def qk_norm_rope_store_and_decode(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_norm_weight: torch.Tensor,
                                   k_norm_weight: torch.Tensor, rope: torch.Tensor, positions: torch.Tensor,
                                   slot_mapping: torch.Tensor, active_mask: torch.Tensor | None,
@@ -165,6 +177,26 @@ def qk_norm_rope_store_and_decode(q: torch.Tensor, k: torch.Tensor, v: torch.Ten
     in the row's table (the decode step's invariant).  Shapes the fused kernel does not cover
     (token row other than 2 KiB, head_dim > 128) run the two launches instead.
     """
+    from .paged_attention import _WORKSPACES
+    o = _fast.prep_decode(q, k, v, q_norm_weight, k_norm_weight, rope, positions, slot_mapping, active_mask, kv_pool,
+                          block_tables, sequence_lengths, layer, eps, scale, out, block_size, max_seq_len, plan,
+                          _WORKSPACES)
+    if o is not None:
+        return o
+    return _qk_norm_rope_store_and_decode(q, k, v, q_norm_weight, k_norm_weight, rope, positions, slot_mapping,
+                                          active_mask, kv_pool, block_tables, sequence_lengths, layer=layer, eps=eps,
+                                          scale=scale, out=out, block_size=block_size, max_seq_len=max_seq_len,
+                                          plan=plan)
+
+
+@accepts_carriers
+def _qk_norm_rope_store_and_decode(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_norm_weight: torch.Tensor,
+                                   k_norm_weight: torch.Tensor, rope: torch.Tensor, positions: torch.Tensor,
+                                   slot_mapping: torch.Tensor, active_mask: torch.Tensor | None,
+                                   kv_pool: torch.Tensor, block_tables: torch.Tensor,
+                                   sequence_lengths: torch.Tensor, *, layer: int = 0, eps: float = 1e-6,
+                                   scale: float | None = None, out: torch.Tensor | None = None,
+                                   block_size: int = 16, max_seq_len: int | None = None, plan=None) -> torch.Tensor:
     from .paged_attention import _check, _plan_key, paged_attention, workspace_for
     from .kv_store import _check_index
     pool_layer, (P, bs, hkv, d) = check_pool(kv_pool, layer, PagedAttentionError)
@@ -255,6 +287,22 @@ def qk_norm_rope_append_and_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.T
     instead.  ``validate``: every table entry the chunk's keys use names a page of the pool
     (checked before the launch; a debug mode that synchronises).
     """
+    if not validate:
+        from .paged_attention import _WORKSPACES
+        o = _fast.prep_prefill(q, k, v, q_norm_weight, k_norm_weight, rope, kv_pool, block_table, query_start, layer,
+                               eps, scale, out, block_size, _WORKSPACES)
+        if o is not None:
+            return o
+    return _qk_norm_rope_append_and_prefill(q, k, v, q_norm_weight, k_norm_weight, rope, kv_pool, block_table,
+                                            query_start=query_start, layer=layer, eps=eps, scale=scale, out=out,
+                                            block_size=block_size, validate=validate)
+
+
+def _qk_norm_rope_append_and_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_norm_weight: torch.Tensor,
+                                     k_norm_weight: torch.Tensor, rope: torch.Tensor, kv_pool: torch.Tensor,
+                                     block_table: torch.Tensor, *, query_start: int, layer: int = 0,
+                                     eps: float = 1e-6, scale: float | None = None, out: torch.Tensor | None = None,
+                                     block_size: int = 16, validate: bool = False) -> torch.Tensor:
     from .paged_attention import _check, _validate_pages, paged_attention, workspace_for
     pool_layer, (P, bs, hkv, d) = check_pool(kv_pool, layer, PagedAttentionError)
     dev = pool_layer.device

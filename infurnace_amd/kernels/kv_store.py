@@ -22,6 +22,7 @@ from __future__ import annotations
 import torch
 
 from .. import _capi
+from . import _fast
 from ._common import KVStoreError, check_pool, current_stream, ptr
 from ._carrier import accepts_carriers
 
@@ -68,7 +69,6 @@ def _debug_validate(slot_mapping: torch.Tensor, active_mask, num_slots: int) -> 
         raise KVStoreError("two active rows map to the same slot")
 
 
-@accepts_carriers
 def store_kv(kv_pool: torch.Tensor, slot_mapping: torch.Tensor, active_mask: torch.Tensor | None,
              new_k: torch.Tensor, new_v: torch.Tensor, *, layer: int = 0, validate: bool = False) -> None:
     """Append ``new_k``/``new_v`` [T, Hkv, D] fp16 into ``kv_pool`` in place.
@@ -78,6 +78,14 @@ def store_kv(kv_pool: torch.Tensor, slot_mapping: torch.Tensor, active_mask: tor
     is int32 [T]; ``active_mask`` is bool/uint8 [T] or None.  ``validate=True``
     adds a synchronising host check for out-of-range and duplicate active slots.
     """
+    if not validate and _fast.store(kv_pool, slot_mapping, active_mask, new_k, new_v, layer) is not None:
+        return None
+    return _store_kv(kv_pool, slot_mapping, active_mask, new_k, new_v, layer=layer, validate=validate)
+
+
+@accepts_carriers
+def _store_kv(kv_pool: torch.Tensor, slot_mapping: torch.Tensor, active_mask: torch.Tensor | None,
+              new_k: torch.Tensor, new_v: torch.Tensor, *, layer: int = 0, validate: bool = False) -> None:
     pool_layer, (P, bs, hkv, d) = check_pool(kv_pool, layer, KVStoreError)
     dev = pool_layer.device
     if not isinstance(new_k, torch.Tensor) or new_k.ndim != 3:
@@ -95,7 +103,6 @@ def store_kv(kv_pool: torch.Tensor, slot_mapping: torch.Tensor, active_mask: tor
                T, hkv, d, bs, current_stream(dev))
 
 
-@accepts_carriers
 def store_kv_layers(kv_pool: torch.Tensor, slot_mapping: torch.Tensor, active_mask: torch.Tensor | None,
                     new_k: torch.Tensor, new_v: torch.Tensor, *, validate: bool = False) -> None:
     """Append one token batch into every layer with a single launch.
@@ -104,6 +111,14 @@ def store_kv_layers(kv_pool: torch.Tensor, slot_mapping: torch.Tensor, active_ma
     mapping and mask are shared by all layers.  Equivalent to ``store_kv`` once
     per layer (the layer loop of model.py:98 with the store of :134-138).
     """
+    if not validate and _fast.store_layers(kv_pool, slot_mapping, active_mask, new_k, new_v) is not None:
+        return None
+    return _store_kv_layers(kv_pool, slot_mapping, active_mask, new_k, new_v, validate=validate)
+
+
+@accepts_carriers
+def _store_kv_layers(kv_pool: torch.Tensor, slot_mapping: torch.Tensor, active_mask: torch.Tensor | None,
+                     new_k: torch.Tensor, new_v: torch.Tensor, *, validate: bool = False) -> None:
     if not isinstance(kv_pool, torch.Tensor) or kv_pool.ndim != 6:
         raise KVStoreError("kv_pool must be the rank-6 [layers, 2, pages, block_size, Hkv, D] pool")
     check_pool(kv_pool, 0, KVStoreError)

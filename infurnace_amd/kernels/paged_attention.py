@@ -25,6 +25,7 @@ import math
 import torch
 
 from .. import _capi
+from . import _fast
 from ._common import PagedAttentionError, check_pool, current_stream, ptr
 from ._carrier import accepts_carriers
 
@@ -231,7 +232,6 @@ def _check(name: str, t, shape: tuple, dtypes: tuple, device) -> None:
         raise PagedAttentionError(f"{name} must be contiguous")
 
 
-@accepts_carriers
 def paged_attention(query: torch.Tensor, kv_pool: torch.Tensor, block_tables: torch.Tensor,
                     sequence_lengths: torch.Tensor | None, active_mask: torch.Tensor | None = None, *,
                     layer: int = 0, scale: float | None = None, query_start: int | None = None,
@@ -270,6 +270,29 @@ def paged_attention(query: torch.Tensor, kv_pool: torch.Tensor, block_tables: to
     must equal query_start + T.  ``active_mask`` of one False row makes the call
     a no-op.
     """
+    if not validate:
+        if query_start is None:
+            o = _fast.decode(query, kv_pool, block_tables, sequence_lengths, active_mask, None, None, None, layer,
+                             scale, out, block_size, max_seq_len, plan, shared_prefix_pages, _WORKSPACES)
+            if o is not None:
+                return o
+        elif sequence_lengths is None and active_mask is None:
+            o = _fast.prefill(query, kv_pool, block_tables, None, None, query_start, layer, scale, out, block_size,
+                              _WORKSPACES)
+            if o is not None:
+                return o
+    return _paged_attention(query, kv_pool, block_tables, sequence_lengths, active_mask, layer=layer, scale=scale,
+                            query_start=query_start, out=out, block_size=block_size, max_seq_len=max_seq_len,
+                            shared_prefix_pages=shared_prefix_pages, plan=plan, validate=validate)
+
+
+@accepts_carriers
+def _paged_attention(query: torch.Tensor, kv_pool: torch.Tensor, block_tables: torch.Tensor,
+                     sequence_lengths: torch.Tensor | None, active_mask: torch.Tensor | None = None, *,
+                     layer: int = 0, scale: float | None = None, query_start: int | None = None,
+                     out: torch.Tensor | None = None, block_size: int = 16,
+                     max_seq_len: int | None = None, shared_prefix_pages: torch.Tensor | None = None,
+                     plan: DecodePlan | None = None, validate: bool = False) -> torch.Tensor:
     pool_layer, (P, bs, hkv, d) = check_pool(kv_pool, layer, PagedAttentionError)
     dev = pool_layer.device
     if bs != block_size:
@@ -391,7 +414,6 @@ def paged_attention(query: torch.Tensor, kv_pool: torch.Tensor, block_tables: to
     return out
 
 
-@accepts_carriers
 def store_kv_and_decode(query: torch.Tensor, kv_pool: torch.Tensor, block_tables: torch.Tensor,
                         sequence_lengths: torch.Tensor, active_mask: torch.Tensor | None,
                         slot_mapping: torch.Tensor, new_k: torch.Tensor, new_v: torch.Tensor, *, layer: int = 0,
@@ -408,6 +430,23 @@ def store_kv_and_decode(query: torch.Tensor, kv_pool: torch.Tensor, block_tables
     ``plan``: the step's ``decode_plan`` built with this ``slot_mapping``.  ``validate`` as for
     ``paged_attention``, plus the slots (as ``store_kv(..., validate=True)``).
     """
+    if not validate and slot_mapping is not None:
+        o = _fast.decode(query, kv_pool, block_tables, sequence_lengths, active_mask, slot_mapping, new_k, new_v, layer,
+                         scale, out, block_size, max_seq_len, plan, None, _WORKSPACES)
+        if o is not None:
+            return o
+    return _store_kv_and_decode(query, kv_pool, block_tables, sequence_lengths, active_mask, slot_mapping, new_k,
+                                new_v, layer=layer, scale=scale, out=out, block_size=block_size,
+                                max_seq_len=max_seq_len, plan=plan, validate=validate)
+
+
+@accepts_carriers
+def _store_kv_and_decode(query: torch.Tensor, kv_pool: torch.Tensor, block_tables: torch.Tensor,
+                         sequence_lengths: torch.Tensor, active_mask: torch.Tensor | None,
+                         slot_mapping: torch.Tensor, new_k: torch.Tensor, new_v: torch.Tensor, *, layer: int = 0,
+                         scale: float | None = None, out: torch.Tensor | None = None, block_size: int = 16,
+                         max_seq_len: int | None = None, plan: DecodePlan | None = None,
+                         validate: bool = False) -> torch.Tensor:
     from .kv_store import _check_index, _check_rows
     if slot_mapping is None:
         raise PagedAttentionError("store_kv_and_decode needs a slot_mapping")
@@ -472,7 +511,6 @@ def store_kv_and_decode(query: torch.Tensor, kv_pool: torch.Tensor, block_tables
     return out
 
 
-@accepts_carriers
 def store_kv_and_prefill(query: torch.Tensor, kv_pool: torch.Tensor, block_table: torch.Tensor, new_k: torch.Tensor,
                          new_v: torch.Tensor, *, query_start: int, layer: int = 0, scale: float | None = None,
                          out: torch.Tensor | None = None, block_size: int = 16, validate: bool = False) -> torch.Tensor:
@@ -485,6 +523,19 @@ def store_kv_and_prefill(query: torch.Tensor, kv_pool: torch.Tensor, block_table
     attention as two launches.  ``validate``: every table entry the chunk's keys use names a page
     of the pool (checked before the launch; a debug mode that synchronises).
     """
+    if not validate and new_k is not None:
+        o = _fast.prefill(query, kv_pool, block_table, new_k, new_v, query_start, layer, scale, out, block_size,
+                          _WORKSPACES)
+        if o is not None:
+            return o
+    return _store_kv_and_prefill(query, kv_pool, block_table, new_k, new_v, query_start=query_start, layer=layer,
+                                 scale=scale, out=out, block_size=block_size, validate=validate)
+
+
+@accepts_carriers
+def _store_kv_and_prefill(query: torch.Tensor, kv_pool: torch.Tensor, block_table: torch.Tensor, new_k: torch.Tensor,
+                          new_v: torch.Tensor, *, query_start: int, layer: int = 0, scale: float | None = None,
+                          out: torch.Tensor | None = None, block_size: int = 16, validate: bool = False) -> torch.Tensor:
     from .kv_store import _check_rows
     pool_layer, (P, bs, hkv, d) = check_pool(kv_pool, layer, PagedAttentionError)
     dev = pool_layer.device

@@ -1,0 +1,45 @@
+"""The wrappers' native argument checks decline what is not theirs (CPU: no call may reach a kernel)."""
+import numpy as np
+import pytest
+import torch
+
+from infurnace_amd.kernels import (KVStoreError, PagedAttentionError, _fast, paged_attention, qk_norm_rope_append,
+                                   store_kv, store_kv_and_decode)
+
+H = torch.float16
+POOL = torch.zeros((2, 4, 16, 8, 128), dtype=H)
+I = torch.zeros(3, dtype=torch.int32)
+Q = torch.zeros((3, 16, 128), dtype=H)
+KV = torch.zeros((3, 8, 128), dtype=H)
+BT = torch.zeros((3, 1), dtype=torch.int32)
+
+
+def test_declines_everything_that_is_no_gpu_tensor():
+    ext = _fast.load()
+    decode = [Q, POOL, BT, I, None, I, KV, KV, 0, None, None, 16, None, None, None, {}]
+    assert ext.decode(*decode) is None
+    for i in range(len(decode)):
+        for odd in (None, 1.5, "x", np.zeros(3), object(), Q.to("meta")):
+            assert ext.decode(*decode[:i], odd, *decode[i + 1:]) is None
+    assert ext.decode() is None and ext.decode(*decode, 1) is None  # wrong counts
+    assert ext.store(POOL, I, None, KV, KV, 0) is None and ext.store_layers(POOL[None], I, None, KV[None], KV[None]) is None
+    assert ext.prefill(Q, POOL, BT[0], None, None, 0, 0, None, None, 16, {}) is None
+    assert ext.prep_append(Q, KV, KV, Q, Q, Q, I, I, None, POOL, 0, 1e-6, None) is None
+    assert ext.prep_decode(*([None] * 20)) is None and ext.prep_prefill(*([None] * 15)) is None
+    with pytest.raises(TypeError):
+        ext.bind(1)
+
+
+def test_errors_are_the_checked_path_s():
+    with pytest.raises(KVStoreError):
+        store_kv(POOL, I, None, KV, KV)
+    with pytest.raises(KVStoreError):
+        store_kv(POOL.float(), I, None, KV, KV)
+    with pytest.raises(PagedAttentionError):
+        paged_attention(Q, POOL, BT, I)
+    with pytest.raises(PagedAttentionError):
+        store_kv_and_decode(Q, POOL, BT, I, None, None, KV, KV)
+    with pytest.raises(KVStoreError):
+        qk_norm_rope_append(Q.float(), KV.float(), KV.float(), Q, Q, Q, I, I, None, POOL)
+    with pytest.raises(TypeError):
+        store_kv(POOL[None], I, None, KV, KV, layer=None)
