@@ -53,8 +53,18 @@ struct WideCfg {
   // unpadded; the 16-byte chunk c of row r sits at chunk position c ^ 2 (r % 4), so the 4 rows a
   // 16-lane group reads in one transposing load fall on disjoint banks.
   static constexpr int kRowChunks = D / 8;                     // 16-byte chunks per key row
-  static constexpr int kHalfInstr = 16 * kRowChunks / kWave;   // DMA instructions per page half
-  static constexpr int kHalfBytes = 16 * D * 2;
+  static constexpr int kHalfInstr = 16 * kRowChunks / kWave;   // 16-byte loads per page half
+  // With 4 waves (kPad) K and V rows are padded instead, so that one LDS cycle -- 16 lanes of a 16-byte
+  // access, 32 of an 8-byte one -- covers the 64 banks once: K rows by 16 bytes (a fragment read takes
+  // one chunk of 16 rows), V rows by 64 (a transposing read takes 64 bytes of 4 rows).  The swizzles
+  // above conflict twofold on K writes and V reads (us, 32 / 8 heads x 128: 512 queries at 6144 81.6 -> 77.0, 333
+  // at 720 19.0 -> 18.2; 16 / 8, 2048 at 0 34.7 -> 33.1; outputs bit-identical).
+  // With 8 waves the constant offsets of padded rows cost registers that the loop does not have.
+  static constexpr bool kPad = W == 4;
+  static constexpr int kRowsInstr = kWave / kRowChunks;        // key rows per 16-byte load instruction
+  static constexpr int kKRowBytes = 2 * D + 16;
+  static constexpr int kVRowBytes = 2 * D + (kPad ? 64 : 0);
+  static constexpr int kHalfBytes = 16 * kVRowBytes;
   static constexpr int kVBufBytes = 2 * kHalfBytes;
   static constexpr int kVInstr = 2 * kHalfInstr;     // 16-byte loads (and LDS writes) per lane per tile
   // V tiles in LDS per wave: i and i + 1 with 4 waves; with 8 (two per SIMD, so half the LDS
@@ -65,7 +75,7 @@ struct WideCfg {
   // four lane bases, and every 8 lanes of a 16-byte write or read (one 128-byte LDS cycle) cover
   // the 32 banks once.
   static constexpr int kKInstr = 32 * kRowChunks / kWave;  // 16-byte loads (and writes) per lane
-  static constexpr int kKBufBytes = 32 * kRowChunks * 16;
+  static constexpr int kKBufBytes = kPad ? 32 * kKRowBytes : 32 * kRowChunks * 16;
   static constexpr int kWaveBytes = kVBufs * kVBufBytes + kKBufBytes;
   static constexpr int kTileBytes = W * kWaveBytes;
   // The queries, staged once per workgroup: kRows rows x D dims, chunk c of row r at c ^ (r % 8).
@@ -310,7 +320,7 @@ __device__ __forceinline__ void prefill_wide_body(
 #pragma unroll
   for (int n = 0; n < C::kHalfInstr; ++n) {
     const int slot = n * kWave + lane, r = slot / C::kRowChunks;
-    const int c = (slot % C::kRowChunks) ^ (2 * (r % 4));
+    const int c = C::kPad ? slot % C::kRowChunks : (slot % C::kRowChunks) ^ (2 * (r % 4));
     voff[n] = uint32_t((r * int(tok_stride) + 8 * c) * 2);
   }
   constexpr int kCB = C::kRowChunks / 8;  // chunk blocks per row
@@ -321,16 +331,21 @@ __device__ __forceinline__ void prefill_wide_body(
 #pragma unroll
     for (int n = 0; n < C::kKInstr / 2; ++n) {
       const int r = 8 * ((n / kCB) % 2) + a, c = 8 * (n % kCB) + e;
-      koff[n] = uint32_t((r * int(tok_stride) + 8 * c) * 2);
+      koff[n] = C::kPad ? voff[n] : uint32_t((r * int(tok_stride) + 8 * c) * 2);
     }
-    kwr = uint32_t((e * 32 + (a ^ e)) * 16);
+    kwr = C::kPad ? uint32_t((lane / C::kRowChunks) * C::kKRowBytes + (lane % C::kRowChunks) * 16)
+                  : uint32_t((e * 32 + (a ^ e)) * 16);
   }
   lds_u8* const vlds = (lds_u8*)(smem) + grp * C::kWaveBytes;
   lds_u8* const klds = vlds + C::kVBufs * C::kVBufBytes;
   // this lane's K fragment of K-step s (key row col, chunk 2 s + half) is at kfrag[s % 4] + 1 KiB s
+  // (padded: at kfrag[0] + 32 s)
   const lds_u8* kfrag[4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) kfrag[j] = klds + half * 512 + (col ^ ((2 * j + half) % 8)) * 16;
+  for (int j = 0; j < 4; ++j)
+    kfrag[j] = C::kPad ? klds + col * C::kKRowBytes + half * 16 : klds + half * 512 + (col ^ ((2 * j + half) % 8)) * 16;
+  const uint32_t vwr = C::kPad ? uint32_t((lane / C::kRowChunks) * C::kVRowBytes + (lane % C::kRowChunks) * 16)
+                               : uint32_t(lane * 16);  // V's LDS write offset of load 0
   struct VTile {
     __amdgpu_buffer_rsrc_t r[2];
     uint32_t add[2];
@@ -364,7 +379,7 @@ __device__ __forceinline__ void prefill_wide_body(
   };
   auto v_store = [&](lds_u8* dst, int j, u32x4 v) __attribute__((always_inline)) {
     const int h = j / C::kHalfInstr, n = j % C::kHalfInstr;
-    *reinterpret_cast<__attribute__((address_space(3))) u32x4*>(dst + h * C::kHalfBytes + (n * kWave + lane) * 16) = v;
+    *reinterpret_cast<__attribute__((address_space(3))) u32x4*>(dst + vwr + h * C::kHalfBytes + n * C::kRowsInstr * C::kVRowBytes) = v;
   };
   // load n (of kKInstr) of a tile's K, its LDS write, and the read of K-step s's fragment
   auto k_load = [&](const VTile& t, int n) __attribute__((always_inline)) {
@@ -374,10 +389,11 @@ __device__ __forceinline__ void prefill_wide_body(
   auto k_store = [&](int n, u32x4 v) __attribute__((always_inline)) {
     const int rb = n / kCB, cb = n % kCB;  // row block (8 rows), chunk block (8 chunks)
     // slot c 32 + (r ^ (c % 8)) = 256 cb + 8 rb + [32 e + (a ^ e)]
-    *reinterpret_cast<__attribute__((address_space(3))) u32x4*>(klds + kwr + cb * 4096 + rb * 128) = v;
+    *reinterpret_cast<__attribute__((address_space(3))) u32x4*>(
+        klds + kwr + (C::kPad ? n * C::kRowsInstr * C::kKRowBytes : cb * 4096 + rb * 128)) = v;
   };
   auto k_read = [&](int s) __attribute__((always_inline)) {
-    return *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(kfrag[s % 4] + 1024 * s);
+    return *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(C::kPad ? kfrag[0] + 32 * s : kfrag[s % 4] + 1024 * s);
   };
 
   // Transposing V reads: lane = 16 g + 4 rr + q reads key row R = 4 (lane / 32) + rr of a page half,
@@ -390,8 +406,8 @@ __device__ __forceinline__ void prefill_wide_body(
     const int b2 = rr / 2;
     const int low = (2 * g2 + q4 / 2) ^ (2 * (rr % 2));
     const int base = (4 * half + rr) * 2 * D + 16 * low + 8 * (q4 % 2);
-    tr_even = base + 64 * b2;
-    tr_odd = base - 64 * b2;
+    tr_even = C::kPad ? (4 * half + rr) * C::kVRowBytes + 32 * g2 + 8 * q4 : base + 64 * b2;
+    tr_odd = C::kPad ? tr_even : base - 64 * b2;
   }
 
   float m[RT], lsum[RT];
@@ -524,7 +540,7 @@ __device__ __forceinline__ void prefill_wide_body(
   auto pv_batch = [&](auto bc, const lds_u8* ae, const lds_u8* ao, const f16x8 (&pb16)[RT][2], auto&& after)
       __attribute__((always_inline)) {
     constexpr int b = decltype(bc)::value;
-    constexpr int d0 = 2 * b, HB = C::kHalfBytes, HI = 16 * D;
+    constexpr int d0 = 2 * b, HB = C::kHalfBytes, HI = 8 * C::kVRowBytes;
     u32x2 rd[8];
     rd[0] = ds_read_tr16(ae + 64 * d0);
     rd[1] = ds_read_tr16(ae + 64 * d0 + HI);
