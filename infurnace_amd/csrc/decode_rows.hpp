@@ -438,10 +438,9 @@ struct RowsMerge {
   __device__ __forceinline__ uint32_t o_off(int64_t s, int qh, int d4) const {
     return uint32_t(((s * HQ + qh) * D + 4 * d4) * (F32 ? 4 : 2));
   }
-  // A state's 4 dims, O (normalised) to slot s.
-  __device__ __forceinline__ void put(int64_t s, int qh, int d4, f32x4 o) const {
-    if constexpr (F32) st_dev4(r_o, o_off(s, qh, d4), o);
-    else st_dev2(r_o, o_off(s, qh, d4), __builtin_bit_cast(f32x2, f16x4{f16(o[0]), f16(o[1]), f16(o[2]), f16(o[3])}));
+  static __device__ __forceinline__ auto state_dims(const State& s) {
+    if constexpr (F32) return s;
+    else return __builtin_bit_cast(f16x4, s);
   }
   // Log-sum-exp merge of a split row's np states (slots slot0 .. slot0 + np - 1, in range order)
   // for query head qh, dims 4 d4 .. 4 d4 + 3.  Every lane loads each state's (m, l) itself (the
@@ -482,15 +481,10 @@ struct RowsMerge {
       for (int u = 0; u < MB; ++u) {
         if (u < cnt) {
           const float w = exp2_fast(ld.ml[u][0] - M) * ld.ml[u][1];  // weight of O / l: e^(m - M) l
-          f32x4 oh;
-          if constexpr (F32) {
-            oh = ld.o[u];
-          } else {
-            const f16x4 h = __builtin_bit_cast(f16x4, ld.o[u]);
-            oh = f32x4{float(h[0]), float(h[1]), float(h[2]), float(h[3])};
-          }
+          const auto oh = state_dims(ld.o[u]);
           L += w;
-          O = f32x4{fmaf(w, oh[0], O[0]), fmaf(w, oh[1], O[1]), fmaf(w, oh[2], O[2]), fmaf(w, oh[3], O[3])};
+          O = f32x4{fmaf(w, float(oh[0]), O[0]), fmaf(w, float(oh[1]), O[1]), fmaf(w, float(oh[2]), O[2]),
+                    fmaf(w, float(oh[3]), O[3])};
         }
       }
     }
@@ -980,8 +974,12 @@ __device__ __forceinline__ void decode_rows_body(
     const int rem = TPW == 1 ? e - a - wave : (e - a + TPW - 1) / TPW - wave;
     const int nw = rem > 0 ? (rem + kRowsWaves - 1) / kRowsWaves : 0;
     auto first_pos = [&](int i) { return a + wave * TPW + kRowsWaves * TPW * i; };
-    auto rel_page = [&](int i) { return first_pos(i) / PB - pg0; };
-    auto page_at = [&](int rp) -> int {
+    auto rel_page = [&](int i) { return (a + wave * TPW + kRowsWaves * TPW * i) / PB - pg0; };
+    auto page_of = [&](int i) -> int {
+      const int rp = rel_page(i);
+      return (rp >> 6) == cur_w ? __builtin_amdgcn_readlane(ids0, rp & 63) : __builtin_amdgcn_readlane(ids1, rp & 63);
+    };
+    auto page_at = [&](int rp) -> int {  // (smaller rows: the page of the last one)
       return (rp >> 6) == cur_w ? __builtin_amdgcn_readlane(ids0, rp & 63) : __builtin_amdgcn_readlane(ids1, rp & 63);
     };
     auto shift = [&](int i) {  // token i's page enters the next 64-page window of the piece
@@ -993,16 +991,17 @@ __device__ __forceinline__ void decode_rows_body(
     };
     // (ok: the token is in the piece and its page in the pool; uniform when TPW == 1)
     auto issue = [&](int i, u32x4 (&kr)[2], u32x4 (&vr)[2], bool& ok) {
-      int p = first_pos(i), phys = page_at(p / PB - pg0);
-      bool in = true;
-      if constexpr (TPW > 1) {  // a wave's rows lie on at most two pages
-        const int p1 = min(p + TPW - 1, e - 1), rp0 = p / PB;
-        const int phys1 = page_at(p1 / PB - pg0);
-        in = p + sub < e;
-        p = min(p + sub, e - 1);
-        phys = p / PB == rp0 ? phys : phys1;
+      int p = first_pos(i);
+      int phys = page_of(i);
+      if constexpr (TPW == 1) {
+        ok = phys >= 0 && int64_t(phys) < num_pages;
+      } else {  // a wave's rows lie on at most two pages; past the piece's end the last one again
+        const int p0 = p;
+        const int phys1 = page_at(min(p0 + TPW - 1, e - 1) / PB - pg0);
+        p = min(p0 + sub, e - 1);
+        phys = p / PB == p0 / PB ? phys : phys1;
+        ok = p0 + sub < e && phys >= 0 && int64_t(phys) < num_pages;
       }
-      ok = phys >= 0 && int64_t(phys) < num_pages;
       const int64_t tok = int64_t(ok ? phys : 0) * PB + p % PB;
       const f16* kb = pool + tok * ROW;
       const f16* vb = pool + v_off + tok * ROW;
@@ -1012,7 +1011,6 @@ __device__ __forceinline__ void decode_rows_body(
           vb = ap.new_v + int64_t(b) * ROW;
         }
       }
-      ok = ok && in;
       kr[0] = kStream ? ld16_stream(kb + off0) : ld16(kb + off0);
       kr[1] = kStream ? ld16_stream(kb + off1) : ld16(kb + off1);
       vr[0] = kStream ? ld16_stream(vb + off0) : ld16(vb + off0);
@@ -1197,7 +1195,12 @@ __device__ __forceinline__ void decode_rows_body(
           mg.write_row(b, qh, d4, M, L, O, kCascade && P.off > 0, pb);
         } else {  // publish this range's state of the row; its ticket is taken at the end
           const float inv = L > 0.f ? 1.f / L : 0.f;
-          mg.put(slot, qh, d4, f32x4{O[0] * inv, O[1] * inv, O[2] * inv, O[3] * inv});
+          if constexpr (kF32) {
+            st_dev4(r_o, mg.o_off(slot, qh, d4), f32x4{O[0] * inv, O[1] * inv, O[2] * inv, O[3] * inv});
+          } else {
+            const f16x4 oh = f16x4{f16(O[0] * inv), f16(O[1] * inv), f16(O[2] * inv), f16(O[3] * inv)};
+            st_dev2(r_o, mg.o_off(slot, qh, d4), __builtin_bit_cast(f32x2, oh));
+          }
           if (d4 == 0) st_dev2(r_ml, mg.ml_off(slot, qh), f32x2{M, L});
         }
       }
