@@ -157,7 +157,20 @@ struct Call {  // the stream and its workspace
   void* stream;
   void* ws;
   size_t bytes;
+  at::Tensor held;  // (another thread may replace the workspace during the launch)
 };
+
+// Calls an entry point without the GIL: a launch can wait for room in the stream's queue, and other threads
+// run meanwhile, as they do in a ctypes call.
+struct NoGil {
+  PyThreadState* state = PyEval_SaveThread();
+  ~NoGil() { PyEval_RestoreThread(state); }
+};
+template <class F, class... A>
+int launch(F fn, A... args) {
+  const NoGil released;
+  return fn(args...);
+}
 
 Call call_on(PyObject* workspaces, int dev, size_t nbytes) {
   Call c;
@@ -171,6 +184,7 @@ Call call_on(PyObject* workspaces, int dev, size_t nbytes) {
   need(size_t(t.numel()) >= nbytes);
   c.ws = t.data_ptr();
   c.bytes = size_t(t.numel());
+  c.held = t;
   return c;
 }
 
@@ -197,6 +211,7 @@ struct Plan {  // a DecodePlan built from this call's tensors (DecodePlan.ptr_fo
   void* p = nullptr;
   size_t bytes = 0;
   bool pending = false;
+  at::Tensor held;
 };
 
 PyObject* attr(PyObject* o, PyObject* name) {  // a new reference
@@ -226,14 +241,15 @@ Plan plan_of(PyObject* o, const Pool& P, int64_t n, int64_t hq, const at::Tensor
   if (ok && buf != Py_None) {
     ok = THPVariable_CheckExact(buf);
     if (ok) {
-      r.p = THPVariable_Unpack(buf).data_ptr();
+      r.held = THPVariable_Unpack(buf);
+      r.p = r.held.data_ptr();
       r.bytes = PyLong_AsSize_t(nb);
     }
   }
   if (ok) r.pending = pend == Py_True;
   Py_XDECREF(nb);
   Py_XDECREF(pend);
-  Py_DECREF(buf);  // (the plan object holds it)
+  Py_DECREF(buf);
   need(ok);
   return r;
 }
@@ -293,23 +309,23 @@ PyObject* decode(PyObject* const* a) {
   const void* qp = q.data_ptr();
   int rc;
   if (shared)
-    rc = E.shared(o, qp, P.p, P.pages, spp, int32_t(sp), tab, mp, sl, act, B, Q, P.hkv, P.d, P.bs, msl, scale, c.ws,
-                  c.bytes, c.stream);
+    rc = launch(E.shared, o, qp, P.p, P.pages, spp, int32_t(sp), tab, mp, sl, act, B, Q, P.hkv, P.d, P.bs, msl, scale,
+                c.ws, c.bytes, c.stream);
   else if (append)
     rc = a[13] == Py_None
-             ? E.decode_append(o, qp, P.p, P.pages, tab, mp, sl, act, slots, nk, nv, B, Q, P.hkv, P.d, P.bs, msl, scale,
-                               c.ws, c.bytes, c.stream)
-         : pl.pending ? E.decode_append_planning(o, qp, P.p, P.pages, tab, mp, sl, act, slots, nk, nv, B, Q, P.hkv, P.d,
-                                                 P.bs, msl, scale, pl.p, pl.bytes, c.ws, c.bytes, c.stream)
-                      : E.decode_append_planned(o, qp, P.p, P.pages, tab, mp, sl, act, slots, nk, nv, B, Q, P.hkv, P.d,
-                                                P.bs, msl, scale, pl.p, pl.bytes, c.ws, c.bytes, c.stream);
+             ? launch(E.decode_append, o, qp, P.p, P.pages, tab, mp, sl, act, slots, nk, nv, B, Q, P.hkv, P.d, P.bs,
+                      msl, scale, c.ws, c.bytes, c.stream)
+         : pl.pending ? launch(E.decode_append_planning, o, qp, P.p, P.pages, tab, mp, sl, act, slots, nk, nv, B, Q,
+                               P.hkv, P.d, P.bs, msl, scale, pl.p, pl.bytes, c.ws, c.bytes, c.stream)
+                      : launch(E.decode_append_planned, o, qp, P.p, P.pages, tab, mp, sl, act, slots, nk, nv, B, Q,
+                               P.hkv, P.d, P.bs, msl, scale, pl.p, pl.bytes, c.ws, c.bytes, c.stream);
   else
-    rc = a[13] == Py_None ? E.decode(o, qp, P.p, P.pages, tab, mp, sl, act, B, Q, P.hkv, P.d, P.bs, msl, scale, c.ws,
-                                     c.bytes, c.stream)
-         : pl.pending     ? E.decode_planning(o, qp, P.p, P.pages, tab, mp, sl, act, B, Q, P.hkv, P.d, P.bs, msl, scale,
-                                              pl.p, pl.bytes, c.ws, c.bytes, c.stream)
-                          : E.decode_planned(o, qp, P.p, P.pages, tab, mp, sl, act, B, Q, P.hkv, P.d, P.bs, msl, scale,
-                                             pl.p, pl.bytes, c.ws, c.bytes, c.stream);
+    rc = a[13] == Py_None ? launch(E.decode, o, qp, P.p, P.pages, tab, mp, sl, act, B, Q, P.hkv, P.d, P.bs, msl,
+                                   scale, c.ws, c.bytes, c.stream)
+         : pl.pending     ? launch(E.decode_planning, o, qp, P.p, P.pages, tab, mp, sl, act, B, Q, P.hkv, P.d, P.bs,
+                                   msl, scale, pl.p, pl.bytes, c.ws, c.bytes, c.stream)
+                          : launch(E.decode_planned, o, qp, P.p, P.pages, tab, mp, sl, act, B, Q, P.hkv, P.d, P.bs,
+                                   msl, scale, pl.p, pl.bytes, c.ws, c.bytes, c.stream);
   need(rc == IFN_OK);
   if (pl.pending) need(PyObject_SetAttr(a[13], s_pending, Py_False) == 0);
   return done(out, a[10]);
@@ -347,11 +363,11 @@ PyObject* prep_decode(PyObject* const* a) {
   const int32_t* tab = static_cast<const int32_t*>(bt.data_ptr());
   const int32_t maxpos = small(rope.size(0));
   const int rc = fn != nullptr
-                     ? fn(out.data_ptr(), qp, k, v, qw, kw, rp, maxpos, pos, slots, P.p, P.pages, tab, mp, sl, act, B, Q,
-                          P.hkv, P.d, P.bs, msl, scale, eps, pl.p, pl.bytes, c.ws, c.bytes, c.stream)
-                     : E.prep_decode(out.data_ptr(), qp, k, v, qw, kw, rp, maxpos, pos, slots, P.p, P.pages, tab, mp, sl,
-                                     act, B, Q, P.hkv, P.d, P.bs, msl, scale, eps, pl.p, pl.bytes, c.ws, c.bytes,
-                                     c.stream);
+                     ? launch(fn, out.data_ptr(), qp, k, v, qw, kw, rp, maxpos, pos, slots, P.p, P.pages, tab, mp, sl,
+                              act, B, Q, P.hkv, P.d, P.bs, msl, scale, eps, pl.p, pl.bytes, c.ws, c.bytes, c.stream)
+                     : launch(E.prep_decode, out.data_ptr(), qp, k, v, qw, kw, rp, maxpos, pos, slots, P.p, P.pages,
+                              tab, mp, sl, act, B, Q, P.hkv, P.d, P.bs, msl, scale, eps, pl.p, pl.bytes, c.ws,
+                              c.bytes, c.stream);
   need(rc == IFN_OK);
   if (pl.pending) need(PyObject_SetAttr(a[18], s_pending, Py_False) == 0);
   return done(out, a[15]);
@@ -383,10 +399,12 @@ PyObject* prefill(PyObject* const* a) {
   const Call c = call_on(a[10], P.dev, E.prefill_ws(T, int32_t(start), Q, P.hkv, P.d, P.bs));
   const at::Tensor out = output(a[8], P, n, hq, false);
   const int32_t* tab = static_cast<const int32_t*>(bt.data_ptr());
-  const int rc = append ? E.prefill_append(out.data_ptr(), q.data_ptr(), P.p, P.pages, tab, small(mp), int32_t(start), T,
-                                           nk, nv, Q, P.hkv, P.d, P.bs, scale, c.ws, c.bytes, c.stream)
-                        : E.prefill(out.data_ptr(), q.data_ptr(), P.p, P.pages, tab, small(mp), int32_t(start), T, Q,
-                                    P.hkv, P.d, P.bs, scale, c.ws, c.bytes, c.stream);
+  void* o = out.data_ptr();
+  const void* qp = q.data_ptr();
+  const int rc = append ? launch(E.prefill_append, o, qp, P.p, P.pages, tab, small(mp), int32_t(start), T, nk, nv, Q,
+                                 P.hkv, P.d, P.bs, scale, c.ws, c.bytes, c.stream)
+                        : launch(E.prefill, o, qp, P.p, P.pages, tab, small(mp), int32_t(start), T, Q, P.hkv, P.d,
+                                 P.bs, scale, c.ws, c.bytes, c.stream);
   need(rc == IFN_OK);
   return done(out, a[8]);
 }
@@ -412,10 +430,10 @@ PyObject* prep_prefill(PyObject* const* a) {
   const int32_t T = small(n), Q = small(hq);
   const Call c = call_on(a[14], P.dev, E.prefill_ws(T, int32_t(start), Q, P.hkv, P.d, P.bs));
   const at::Tensor out = output(a[12], P, n, hq, false);
-  const int rc = E.prep_prefill(out.data_ptr(), static_cast<const float*>(q.data_ptr()), k, v, qw, kw,
-                                static_cast<const float*>(rope.data_ptr()), small(rope.size(0)), P.p, P.pages,
-                                static_cast<const int32_t*>(bt.data_ptr()), small(mp), int32_t(start), T, Q, P.hkv, P.d,
-                                P.bs, eps, scale, c.ws, c.bytes, c.stream);
+  const int rc = launch(E.prep_prefill, out.data_ptr(), static_cast<const float*>(q.data_ptr()), k, v, qw, kw,
+                        static_cast<const float*>(rope.data_ptr()), small(rope.size(0)), P.p, P.pages,
+                        static_cast<const int32_t*>(bt.data_ptr()), small(mp), int32_t(start), T, Q, P.hkv, P.d,
+                        P.bs, eps, scale, c.ws, c.bytes, c.stream);
   need(rc == IFN_OK);
   return done(out, a[12]);
 }
@@ -438,9 +456,9 @@ PyObject* prep_append(PyObject* const* a) {
   const uint8_t* act = mask(a[8], P.dev, n);
   const float eps = eps_of(a[11]);
   const at::Tensor out = output(a[12], P, n, hq, false);
-  const int rc = E.prep_append(out.data_ptr(), static_cast<const float*>(q.data_ptr()), k, v, qw, kw,
-                               static_cast<const float*>(rope.data_ptr()), small(rope.size(0)), pos, slots, act, P.p,
-                               P.pages, small(n), small(hq), P.hkv, P.d, P.bs, eps, stream_of(P.dev));
+  const int rc = launch(E.prep_append, out.data_ptr(), static_cast<const float*>(q.data_ptr()), k, v, qw, kw,
+                        static_cast<const float*>(rope.data_ptr()), small(rope.size(0)), pos, slots, act, P.p,
+                        P.pages, small(n), small(hq), P.hkv, P.d, P.bs, eps, stream_of(P.dev));
   need(rc == IFN_OK);
   return done(out, a[12]);
 }
@@ -453,8 +471,8 @@ PyObject* store(PyObject* const* a) {
   const int64_t n = k.size(0);
   shaped(a[3], at::kHalf, P.dev, n, P.hkv, P.d);
   const at::Tensor& v = shaped(a[4], at::kHalf, P.dev, n, P.hkv, P.d);
-  need(E.store_kv(P.p, P.pages, i32(a[1], P.dev, n), mask(a[2], P.dev, n), k.data_ptr(), v.data_ptr(), small(n), P.hkv,
-                  P.d, P.bs, stream_of(P.dev)) == IFN_OK);
+  need(launch(E.store_kv, P.p, P.pages, i32(a[1], P.dev, n), mask(a[2], P.dev, n), k.data_ptr(), v.data_ptr(),
+              small(n), P.hkv, P.d, P.bs, stream_of(P.dev)) == IFN_OK);
   Py_RETURN_TRUE;
 }
 
@@ -466,8 +484,8 @@ PyObject* store_layers(PyObject* const* a) {
   const int64_t n = k.size(1);
   shaped(a[3], at::kHalf, P.dev, P.layers, n, P.hkv, P.d);
   const at::Tensor& v = shaped(a[4], at::kHalf, P.dev, P.layers, n, P.hkv, P.d);
-  need(E.store_kv_layers(P.p, small(P.layers), P.pages, i32(a[1], P.dev, n), mask(a[2], P.dev, n), k.data_ptr(),
-                         v.data_ptr(), small(n), P.hkv, P.d, P.bs, stream_of(P.dev)) == IFN_OK);
+  need(launch(E.store_kv_layers, P.p, small(P.layers), P.pages, i32(a[1], P.dev, n), mask(a[2], P.dev, n), k.data_ptr(),
+              v.data_ptr(), small(n), P.hkv, P.d, P.bs, stream_of(P.dev)) == IFN_OK);
   Py_RETURN_TRUE;
 }
 
