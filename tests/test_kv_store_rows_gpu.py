@@ -15,8 +15,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("hkv,d,layers,tokens",
                          [(4, 128, 1, t) for t in (1, 2, 3, 130)] + [(2, 128, 1, t) for t in (1, 4, 5, 127)]
                          + [(8, 64, 3, 17), (4, 64, 2, 18), (1, 256, 1, 3),
-                            (8, 128, 4, 1025), (8, 128, 20, 1001), (4, 128, 4, 2049), (8, 64, 4, 2047), (4, 128, 4, 2055),
-                            (2, 128, 8, 2049), (2, 128, 8, 2063)])
+                            (8, 128, 4, 1025), (8, 128, 20, 1001), (4, 128, 4, 2049), (8, 64, 4, 2047),
+                            (4, 128, 4, 2055), (2, 128, 8, 2049), (2, 128, 8, 2063)])
 def test_rows_bit_exact(dev, hkv, d, layers, tokens):
     say(f"store rows hkv={hkv} d={d} layers={layers} tokens={tokens}")
     rng = np.random.default_rng(hkv * d + tokens)
