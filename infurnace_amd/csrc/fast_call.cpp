@@ -205,7 +205,7 @@ bool is_tuple(PyObject* o, std::initializer_list<int64_t> v) {
   return true;
 }
 
-PyObject *s_buf, *s_nbytes, *s_pending, *s_key;
+PyObject *s_buf, *s_nbytes, *s_pending, *s_key, *s_slots;
 
 struct Plan {  // a DecodePlan built from this call's tensors (DecodePlan.ptr_for)
   void* p = nullptr;
@@ -252,6 +252,11 @@ Plan plan_of(PyObject* o, const Pool& P, int64_t n, int64_t hq, const at::Tensor
   Py_DECREF(buf);
   need(ok);
   return r;
+}
+
+void plan_built(PyObject* plan, bool slots) {  // DecodePlan.built of a pending plan
+  need(PyObject_SetAttr(plan, s_slots, slots ? Py_True : Py_False) == 0 &&
+       PyObject_SetAttr(plan, s_pending, Py_False) == 0);
 }
 
 int64_t cap_of(PyObject* msl, int64_t cap) {
@@ -327,7 +332,7 @@ PyObject* decode(PyObject* const* a) {
                           : launch(E.decode_planned, o, qp, P.p, P.pages, tab, mp, sl, act, B, Q, P.hkv, P.d, P.bs,
                                    msl, scale, pl.p, pl.bytes, c.ws, c.bytes, c.stream);
   need(rc == IFN_OK);
-  if (pl.pending) need(PyObject_SetAttr(a[13], s_pending, Py_False) == 0);
+  if (pl.pending) plan_built(a[13], append);
   return done(out, a[10]);
 }
 
@@ -369,7 +374,7 @@ PyObject* prep_decode(PyObject* const* a) {
                               tab, mp, sl, act, B, Q, P.hkv, P.d, P.bs, msl, scale, eps, pl.p, pl.bytes, c.ws,
                               c.bytes, c.stream);
   need(rc == IFN_OK);
-  if (pl.pending) need(PyObject_SetAttr(a[18], s_pending, Py_False) == 0);
+  if (pl.pending) plan_built(a[18], true);
   return done(out, a[15]);
 }
 
@@ -537,6 +542,8 @@ PyMODINIT_FUNC PyInit__fast_call() {
   s_nbytes = PyUnicode_InternFromString("nbytes");
   s_pending = PyUnicode_InternFromString("pending");
   s_key = PyUnicode_InternFromString("key");
-  if (s_buf == nullptr || s_nbytes == nullptr || s_pending == nullptr || s_key == nullptr) return nullptr;
+  s_slots = PyUnicode_InternFromString("slots");
+  for (PyObject* s : {s_buf, s_nbytes, s_pending, s_key, s_slots})
+    if (s == nullptr) return nullptr;
   return PyModule_Create(&module);
 }

@@ -267,7 +267,7 @@ def _qk_norm_rope_store_and_decode(q: torch.Tensor, k: torch.Tensor, v: torch.Te
                                out=out, block_size=block_size, max_seq_len=max_seq_len, plan=plan)
     _capi.check("ifn_paged_decode_prep_append", status)
     if plan is not None:
-        plan.built()
+        plan.built(True)
     return out
 
 

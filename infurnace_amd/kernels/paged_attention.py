@@ -65,20 +65,22 @@ class DecodePlan:
     A lazy plan (``decode_plan(..., lazy=True)``) is built by the first decode call
     that takes it (``ifn_paged_decode_planning`` and its append / pre-append forms):
     that call decodes unplanned and writes the plan, so the step needs no plan
-    launch of its own.  It takes the form of that call: built by a call without
-    slots, it serves the fused-append calls only as an unplanned split.
+    launch of its own.  It takes the form of that call (``slots``: the plan holds
+    the appended slots): built by a call without slots, it serves the fused-append
+    calls only as an unplanned split.
     """
 
     def __init__(self, buf, nbytes: int, key: tuple, rebuild=None, pending: bool = False):
         self.buf, self.nbytes, self.key, self._rebuild = buf, nbytes, key, rebuild
         self.pending = pending and buf is not None
+        self.slots = key[1] is not None
 
     def check_current(self) -> None:
         """Validate mode: raise unless a plan built now from the same tensors is identical
         (their contents were not changed since this one was built)."""
         if self.buf is None or self._rebuild is None or self.pending:
             return
-        fresh = self._rebuild()
+        fresh = self._rebuild(self.slots)
         if not torch.equal(fresh.buf, self.buf):
             raise PagedAttentionError("stale DecodePlan: the tables, lengths, mask or slots it was built from "
                                       "have changed since; build a new plan for this step")
@@ -95,9 +97,10 @@ class DecodePlan:
         """The C entry point for the next call: ``planning`` while the plan is still to be built."""
         return planning if self.pending else planned
 
-    def built(self) -> None:
-        """The call that builds a lazy plan has been enqueued."""
-        self.pending = False
+    def built(self, slots: bool) -> None:
+        """A call with the plan has been enqueued; a lazy plan's first one built it, with the step's slots or without."""
+        if self.pending:
+            self.slots, self.pending = slots, False
 
 
 def _plan_key(query_shape, slot_mapping, pool_layer, block_tables, sequence_lengths, active_mask, max_seq_len,
@@ -169,9 +172,9 @@ def decode_plan(query_shape, kv_pool: torch.Tensor, block_tables: torch.Tensor, 
     # (the kernels write every word of a plan; a shared-prefix plan is left alone for some shapes)
     buf = (torch.zeros if sp else torch.empty)(nbytes, dtype=torch.uint8, device=dev)
 
-    def rebuild():
-        return decode_plan(query_shape, kv_pool, block_tables, sequence_lengths, active_mask, slot_mapping,
-                           layer=layer, block_size=block_size, max_seq_len=max_seq_len,
+    def rebuild(slots):
+        return decode_plan(query_shape, kv_pool, block_tables, sequence_lengths, active_mask,
+                           slot_mapping if slots else None, layer=layer, block_size=block_size, max_seq_len=max_seq_len,
                            shared_prefix_pages=shared_prefix_pages)
     if lazy:
         return DecodePlan(buf, nbytes, key, rebuild, pending=True)
@@ -370,7 +373,7 @@ def _paged_attention(query: torch.Tensor, kv_pool: torch.Tensor, block_tables: t
             _capi.call(plan.entry("ifn_paged_decode_planned", "ifn_paged_decode_planning"), ptr(out), ptr(query),
                        ptr(pool_layer), P, ptr(block_tables), max_pages, ptr(sequence_lengths), ptr(active_mask), n,
                        hq, hkv, d, bs, msl, float(scale), pp, plan.nbytes if pp else 0, ptr(ws), ws.numel(), stream)
-            plan.built()
+            plan.built(False)
             return out
         _capi.call("ifn_paged_decode", ptr(out), ptr(query), ptr(pool_layer), P, ptr(block_tables),
                    max_pages, ptr(sequence_lengths), ptr(active_mask), n, hq, hkv, d, bs, msl,
@@ -503,7 +506,7 @@ def _store_kv_and_decode(query: torch.Tensor, kv_pool: torch.Tensor, block_table
                    ptr(query), ptr(pool_layer), P, ptr(block_tables), max_pages, ptr(sequence_lengths),
                    ptr(active_mask), ptr(sm), ptr(new_k), ptr(new_v), n, hq, hkv, d, bs, msl, float(scale), pp,
                    plan.nbytes if pp else 0, ptr(ws), ws.numel(), stream)
-        plan.built()
+        plan.built(True)
         return out
     _capi.call("ifn_paged_decode_append", ptr(out), ptr(query), ptr(pool_layer), P, ptr(block_tables), max_pages,
                ptr(sequence_lengths), ptr(active_mask), ptr(sm), ptr(new_k), ptr(new_v), n, hq, hkv, d, bs, msl,

@@ -11,7 +11,8 @@ import torch
 import oracle
 from gpu_util import assert_attn_close, say, to_dev
 from infurnace_amd import _capi
-from infurnace_amd.kernels import paged_attention, store_kv_and_decode
+from infurnace_amd.kernels import (PagedAttentionError, decode_plan, paged_attention, qk_norm_rope_store_and_decode,
+                                   rope_table, store_kv_and_decode)
 from infurnace_amd.kernels.paged_attention import workspace_for
 from test_decode_planning_gpu import _case, _check
 
@@ -110,3 +111,35 @@ def test_shard_calls_without_a_plan_buffer(dev):
                       nbytes, ws.data_ptr(), ws.numel(), st) == 0
             assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
     assert int(buf.sum()) == 0
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(16, 4, 128), (8, 2, 128), (16, 8, 128)])
+@pytest.mark.parametrize("first", ["prep", "plain"])
+def test_lazy_plan_with_slots_across_call_forms(dev, hq, hkv, d, first):
+    """A lazy plan with slots whose first call takes none (the pre-append step of these rows attends after a
+    separate append): it stays valid for every later call, and is stale only once its tensors change."""
+    say(f"lazy plan across forms hq={hq} hkv={hkv} first={first}")
+    rng = np.random.default_rng(hq + hkv)
+    pool, table, lens, q = _case(rng, [300, 1, 33, 700], hq, hkv, d)
+    qd, p, bt, sl = (to_dev(x, dev) for x in (q, pool, table, lens))
+    pos = lens - 1
+    sm = to_dev((table[np.arange(4), pos // 16] * 16 + pos % 16).astype(np.int32), dev)
+    f = lambda *s: torch.randn(s, device=dev)
+    qf, kf, vf, w = f(4, hq, d), f(4, hkv, d), f(4, hkv, d), f(d)
+    rope, pd = rope_table(700, d, 1e6, device=dev), to_dev(pos.astype(np.int32), dev)
+    plan = decode_plan(qd.shape, p, bt, sl, None, sm, lazy=True)
+    assert plan.pending
+    prep = lambda pl: qk_norm_rope_store_and_decode(qf, kf, vf, w, w, rope, pd, sm, None, p, bt, sl, plan=pl)
+    plain = lambda pl, **o: paged_attention(qd, p, bt, sl, plan=pl, **o)
+    append = lambda pl, **o: store_kv_and_decode(qd, p, bt, sl, None, sm, kf.half(), vf.half(), plan=pl, **o)
+    same = lambda a, b: torch.equal(a.view(torch.int16), b.view(torch.int16))
+    (prep if first == "prep" else plain)(plan)
+    assert not plan.pending
+    assert same(prep(plan), prep(None))
+    for o in ({}, dict(validate=True)):
+        assert same(plain(plan, **o), plain(None))
+        assert same(append(plan, **o), append(None))
+    sl[0] -= 17
+    for call in (plain, append):
+        with pytest.raises(PagedAttentionError, match="stale"):
+            call(plan, validate=True)
