@@ -4,9 +4,10 @@
 // launches.  Each function here makes the wrapper's checks on plain torch tensors and calls the same C
 // entry point.  It handles exactly the calls the checked Python path accepts in its common form and
 // returns None for everything else -- an argument that is no plain contiguous torch tensor, a value out
-// of range, a plan for other tensors, a workspace to grow, a call the entry point refuses -- before
-// anything is launched; the wrapper then takes the Python path, which raises or handles it.  Nothing is
-// kept between calls but the entry points' addresses.
+// of range, a plan for other tensors, a workspace to grow, a call the entry point refuses -- before the
+// entry point launches anything (an output cleared for a call that is then refused is dropped); the wrapper
+// then takes the Python path, which raises or handles it.  A launch that failed is raised here, not made
+// again.  Nothing is kept between calls but the entry points' addresses.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -49,6 +50,7 @@ Entries E{};
 bool bound = false;
 
 struct NotPlain {};  // the call goes to the Python path
+struct Raised {};    // a Python error is set: it goes to the caller
 
 inline void need(bool ok) {
   if (!ok) throw NotPlain{};
@@ -170,6 +172,19 @@ template <class F, class... A>
 int launch(F fn, A... args) {
   const NoGil released;
   return fn(args...);
+}
+
+// An entry point's status.  It refuses a call before it launches anything: that call goes to the Python path.
+// IFN_ERR_HIP is a launch that failed, possibly after another one of the same call: _capi.check raises it.
+void launched(int rc, const char* name) {
+  need(rc == IFN_OK || rc == IFN_ERR_HIP);
+  if (rc == IFN_OK) return;
+  PyObject* capi = PyImport_ImportModule("infurnace_amd._capi");
+  PyObject* r = capi == nullptr ? nullptr : PyObject_CallMethod(capi, "check", "si", name, rc);
+  Py_XDECREF(r);
+  Py_XDECREF(capi);
+  if (r != nullptr) PyErr_SetString(PyExc_RuntimeError, name);
+  throw Raised{};
 }
 
 Call call_on(PyObject* workspaces, int dev, size_t nbytes) {
@@ -331,7 +346,7 @@ PyObject* decode(PyObject* const* a) {
                                    msl, scale, pl.p, pl.bytes, c.ws, c.bytes, c.stream)
                           : launch(E.decode_planned, o, qp, P.p, P.pages, tab, mp, sl, act, B, Q, P.hkv, P.d, P.bs,
                                    msl, scale, pl.p, pl.bytes, c.ws, c.bytes, c.stream);
-  need(rc == IFN_OK);
+  launched(rc, shared ? "ifn_paged_decode_shared_prefix" : append ? "ifn_paged_decode_append" : "ifn_paged_decode");
   if (pl.pending) plan_built(a[13], append);
   return done(out, a[10]);
 }
@@ -373,7 +388,7 @@ PyObject* prep_decode(PyObject* const* a) {
                      : launch(E.prep_decode, out.data_ptr(), qp, k, v, qw, kw, rp, maxpos, pos, slots, P.p, P.pages,
                               tab, mp, sl, act, B, Q, P.hkv, P.d, P.bs, msl, scale, eps, pl.p, pl.bytes, c.ws,
                               c.bytes, c.stream);
-  need(rc == IFN_OK);
+  launched(rc, "ifn_paged_decode_prep_append");
   if (pl.pending) plan_built(a[18], true);
   return done(out, a[15]);
 }
@@ -410,7 +425,7 @@ PyObject* prefill(PyObject* const* a) {
                                  P.hkv, P.d, P.bs, scale, c.ws, c.bytes, c.stream)
                         : launch(E.prefill, o, qp, P.p, P.pages, tab, small(mp), int32_t(start), T, Q, P.hkv, P.d,
                                  P.bs, scale, c.ws, c.bytes, c.stream);
-  need(rc == IFN_OK);
+  launched(rc, append ? "ifn_paged_prefill_append" : "ifn_paged_prefill");
   return done(out, a[8]);
 }
 
@@ -439,7 +454,7 @@ PyObject* prep_prefill(PyObject* const* a) {
                         static_cast<const float*>(rope.data_ptr()), small(rope.size(0)), P.p, P.pages,
                         static_cast<const int32_t*>(bt.data_ptr()), small(mp), int32_t(start), T, Q, P.hkv, P.d,
                         P.bs, eps, scale, c.ws, c.bytes, c.stream);
-  need(rc == IFN_OK);
+  launched(rc, "ifn_paged_prefill_prep_append");
   return done(out, a[12]);
 }
 
@@ -464,7 +479,7 @@ PyObject* prep_append(PyObject* const* a) {
   const int rc = launch(E.prep_append, out.data_ptr(), static_cast<const float*>(q.data_ptr()), k, v, qw, kw,
                         static_cast<const float*>(rope.data_ptr()), small(rope.size(0)), pos, slots, act, P.p,
                         P.pages, small(n), small(hq), P.hkv, P.d, P.bs, eps, stream_of(P.dev));
-  need(rc == IFN_OK);
+  launched(rc, "ifn_qk_norm_rope_append");
   return done(out, a[12]);
 }
 
@@ -476,8 +491,8 @@ PyObject* store(PyObject* const* a) {
   const int64_t n = k.size(0);
   shaped(a[3], at::kHalf, P.dev, n, P.hkv, P.d);
   const at::Tensor& v = shaped(a[4], at::kHalf, P.dev, n, P.hkv, P.d);
-  need(launch(E.store_kv, P.p, P.pages, i32(a[1], P.dev, n), mask(a[2], P.dev, n), k.data_ptr(), v.data_ptr(),
-              small(n), P.hkv, P.d, P.bs, stream_of(P.dev)) == IFN_OK);
+  launched(launch(E.store_kv, P.p, P.pages, i32(a[1], P.dev, n), mask(a[2], P.dev, n), k.data_ptr(), v.data_ptr(),
+                  small(n), P.hkv, P.d, P.bs, stream_of(P.dev)), "ifn_store_kv");
   Py_RETURN_TRUE;
 }
 
@@ -489,12 +504,12 @@ PyObject* store_layers(PyObject* const* a) {
   const int64_t n = k.size(1);
   shaped(a[3], at::kHalf, P.dev, P.layers, n, P.hkv, P.d);
   const at::Tensor& v = shaped(a[4], at::kHalf, P.dev, P.layers, n, P.hkv, P.d);
-  need(launch(E.store_kv_layers, P.p, small(P.layers), P.pages, i32(a[1], P.dev, n), mask(a[2], P.dev, n), k.data_ptr(),
-              v.data_ptr(), small(n), P.hkv, P.d, P.bs, stream_of(P.dev)) == IFN_OK);
+  launched(launch(E.store_kv_layers, P.p, small(P.layers), P.pages, i32(a[1], P.dev, n), mask(a[2], P.dev, n),
+                  k.data_ptr(), v.data_ptr(), small(n), P.hkv, P.d, P.bs, stream_of(P.dev)), "ifn_store_kv_layers");
   Py_RETURN_TRUE;
 }
 
-// A call of N arguments: None when it is not one for this path (no exception leaves it).
+// A call of N arguments: None when it is not one for this path (no C++ exception leaves it).
 template <PyObject* (*F)(PyObject* const*), Py_ssize_t N>
 PyObject* guarded(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (n == N && bound && !at::impl::torch_function_mode_enabled() &&
@@ -502,6 +517,8 @@ PyObject* guarded(PyObject*, PyObject* const* args, Py_ssize_t n) {
     try {
       PyObject* r = F(args);
       if (r != nullptr) return r;
+    } catch (const Raised&) {
+      return nullptr;
     } catch (...) {
     }
     PyErr_Clear();

@@ -1,9 +1,9 @@
 """Native forms of the wrappers' checks and calls (csrc/fast_call.cpp).
 
-Each function takes a wrapper's arguments in order, and either makes the call and returns its result or
-returns None with nothing launched: the arguments are then for the checked Python path, which
-accepts more forms (array carriers, host values) and raises the errors.  Without the extension every
-call takes that path.
+Each function takes a wrapper's arguments in order, and either makes the call and returns its result (a
+launch that fails raises, as on the Python path) or returns None before the entry point launches anything:
+the arguments are then for the checked Python path, which accepts more forms (array carriers, host values)
+and raises the errors.  Without the extension every call takes that path.
 """
 from __future__ import annotations
 

@@ -1,10 +1,12 @@
 """Native wrapper calls against the checked Python path: same results, same refusals."""
+import ctypes
 import sys
 
 import pytest
 import torch
 
 from gpu_util import say
+from infurnace_amd import _capi
 from infurnace_amd.kernels import _fast, decode_plan, kv_prep, kv_store, rope_table
 from infurnace_amd.kernels import KVStoreError, PagedAttentionError, DeviceArray
 
@@ -155,3 +157,49 @@ def test_native_call_uses_the_current_stream(dev):
     s.synchronize()
     assert torch.equal(o.view(torch.int16), ref.view(torch.int16))
     assert (dev.index or 0, s.cuda_stream) in att._WORKSPACES
+
+
+def test_failed_launch_raises_once(dev):
+    """An entry point that reports a failed launch is not called again: its error reaches the caller.  (The
+    entries stand in on the host; nothing is launched.)"""
+    say("native failed launch")
+    t = _Data(dev)
+    wrappers = [lambda: att._paged_attention(t.q, t.pool, t.table, t.lens),
+                lambda: att._paged_attention(t.q, t.pool, t.table[0], None, query_start=32)]
+    for w in wrappers:  # (the workspace is there)
+        w()
+    torch.cuda.synchronize()
+    calls = []
+    status = _capi.IFN_ERR_HIP
+
+    @ctypes.CFUNCTYPE(ctypes.c_int)
+    def failing():
+        calls.append(1)
+        return status
+    lib = _capi.lib()
+    at = [ctypes.cast(failing if not n.endswith("_bytes") else getattr(lib, n), ctypes.c_void_p).value
+          for n in _fast._ENTRIES]
+    each = [lambda: att.paged_attention(t.q, t.pool, t.table, t.lens),
+            lambda: att.store_kv_and_decode(t.q, t.pool, t.table, t.lens, None, t.slots, t.k, t.v),
+            lambda: kv_prep.qk_norm_rope_store_and_decode(t.qf, t.kf, t.vf, t.qw, t.kw, t.rope, t.pos, t.slots, t.act,
+                                                          t.pool, t.table, t.lens),
+            lambda: att.paged_attention(t.q, t.pool, t.table[0], None, query_start=32),
+            lambda: att.store_kv_and_prefill(t.q, t.pool, t.table[0], t.k, t.v, query_start=32),
+            lambda: kv_prep.qk_norm_rope_append_and_prefill(t.qf, t.kf, t.vf, t.qw, t.kw, t.rope, t.pool, t.table[0],
+                                                            query_start=32),
+            lambda: kv_prep.qk_norm_rope_append(t.qf, t.kf, t.vf, t.qw, t.kw, t.rope, t.pos, t.slots, None, t.pool),
+            lambda: kv_store.store_kv(t.pool, t.slots, None, t.k, t.v),
+            lambda: kv_store.store_kv_layers(t.pool, t.slots, None, torch.stack([t.k] * 2), torch.stack([t.v] * 2))]
+    ext = _fast.load()
+    try:
+        ext.bind(*at)
+        for fn in each:
+            del calls[:]
+            with pytest.raises(_capi.KernelLaunchError) as e:
+                fn()
+            assert e.value.status == status and len(calls) == 1
+        status = _capi.IFN_ERR_WORKSPACE  # (a refusal: the checked path makes the call)
+        ref = att._paged_attention(t.q, t.pool, t.table, t.lens)
+        assert torch.equal(each[0]().view(torch.int16), ref.view(torch.int16))
+    finally:
+        _fast.load()
