@@ -148,11 +148,27 @@ float eps_of(PyObject* o) {
   return float(e);
 }
 
+// Work on the device runs without the GIL: a launch (or an output's fill) can wait for room in the stream's
+// queue, an allocation for the device, and other threads run meanwhile, as they do in a ctypes or torch call.
+struct NoGil {
+  PyThreadState* state = PyEval_SaveThread();
+  ~NoGil() { PyEval_RestoreThread(state); }
+};
+template <class F>
+auto unlocked(F f) {
+  const NoGil released;
+  return f();
+}
+template <class F, class... A>
+int launch(F fn, A... args) {
+  return unlocked([&] { return fn(args...); });
+}
+
 // The fp16 output [n, hq, d]: the caller's, or a new one (cleared when rows may be inactive).
 at::Tensor output(PyObject* o, const Pool& P, int64_t n, int64_t hq, bool clear) {
   if (o != Py_None) return shaped(o, at::kHalf, P.dev, n, hq, P.d);
   const auto opt = at::TensorOptions().dtype(at::kHalf).device(at::kCUDA, P.dev);
-  return clear ? at::zeros({n, hq, P.d}, opt) : at::empty({n, hq, P.d}, opt);
+  return unlocked([&] { return clear ? at::zeros({n, hq, P.d}, opt) : at::empty({n, hq, P.d}, opt); });
 }
 
 struct Call {  // the stream and its workspace
@@ -161,18 +177,6 @@ struct Call {  // the stream and its workspace
   size_t bytes;
   at::Tensor held;  // (another thread may replace the workspace during the launch)
 };
-
-// Calls an entry point without the GIL: a launch can wait for room in the stream's queue, and other threads
-// run meanwhile, as they do in a ctypes call.
-struct NoGil {
-  PyThreadState* state = PyEval_SaveThread();
-  ~NoGil() { PyEval_RestoreThread(state); }
-};
-template <class F, class... A>
-int launch(F fn, A... args) {
-  const NoGil released;
-  return fn(args...);
-}
 
 // An entry point's status.  It refuses a call before it launches anything: that call goes to the Python path.
 // IFN_ERR_HIP is a launch that failed, possibly after another one of the same call: _capi.check raises it.

@@ -1,8 +1,12 @@
 """The wrappers' native argument checks decline what is not theirs (CPU: no call may reach a kernel)."""
+import os
+import re
+
 import numpy as np
 import pytest
 import torch
 
+from infurnace_amd.build import CSRC
 from infurnace_amd.kernels import (KVStoreError, PagedAttentionError, _fast, paged_attention, qk_norm_rope_append,
                                    store_kv, store_kv_and_decode)
 
@@ -43,3 +47,12 @@ def test_errors_are_the_checked_path_s():
         qk_norm_rope_append(Q.float(), KV.float(), KV.float(), Q, Q, Q, I, I, None, POOL)
     with pytest.raises(TypeError):
         store_kv(POOL[None], I, None, KV, KV, layer=None)
+
+
+def test_device_work_leaves_the_gil():
+    """Whatever can wait for the device -- an entry point, an output's allocation and fill -- runs without the GIL:
+    a full queue behind a host function that needs it would otherwise never drain."""
+    src = open(os.path.join(CSRC, "fast_call.cpp")).read()
+    work = re.findall(r"at::(?:zeros|empty)\(|\bE\.\w+(?=, )", src)
+    out = re.sub(r"(?:unlocked|launch)\((?:[^()]|\((?:[^()]|\([^()]*\))*\))*\)", "", src)
+    assert len(work) > 12 and re.findall(r"at::(?:zeros|empty)\(|\bE\.\w+(?=, )", out) == []
