@@ -30,6 +30,7 @@ struct Entries {
   decltype(&ifn_store_kv) store_kv;
   decltype(&ifn_store_kv_layers) store_kv_layers;
   decltype(&ifn_paged_decode_workspace_bytes) decode_ws;
+  decltype(&ifn_paged_decode_plan_bytes) plan_bytes;
   decltype(&ifn_paged_decode) decode;
   decltype(&ifn_paged_decode_append) decode_append;
   decltype(&ifn_paged_decode_planned) decode_planned;
@@ -377,6 +378,9 @@ PyObject* prep_decode(PyObject* const* a) {
   const int32_t* sl = i32(a[11], P.dev, n);
   const float eps = eps_of(a[13]), scale = scale_of(a[14], P.d);
   const int32_t msl = small(cap_of(a[17], bt.size(1) * P.bs)), B = small(n), Q = small(hq), mp = small(bt.size(1));
+  // What the fused kernel does not take is declined before an output is made: it takes the calls of the whole-row
+  // kernel (those that have a plan) with 2 KiB token rows, 16-token pages and head dims up to 128.
+  need(P.hkv * P.d == 1024 && P.d <= 128 && P.bs == 16 && E.plan_bytes(B, Q, P.hkv, P.d, P.bs, mp, msl) > 0);
   Plan pl;
   if (a[18] != Py_None) pl = plan_of(a[18], P, n, hq, bt, sl, act, slots, msl);
   const Call c = call_on(a[19], P.dev, E.decode_ws(B, Q, P.hkv, P.d, P.bs, msl));

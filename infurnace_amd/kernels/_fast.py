@@ -16,7 +16,8 @@ from .. import _capi
 EXT_PATH = os.path.join(os.path.dirname(_capi.LIB_PATH), "_fast_call.so")
 _NAMES = ("decode", "prep_decode", "prefill", "prep_prefill", "prep_append", "store", "store_layers")
 # the C entry points the extension calls, in the order it takes their addresses
-_ENTRIES = ("ifn_store_kv", "ifn_store_kv_layers", "ifn_paged_decode_workspace_bytes", "ifn_paged_decode",
+_ENTRIES = ("ifn_store_kv", "ifn_store_kv_layers", "ifn_paged_decode_workspace_bytes",
+            "ifn_paged_decode_plan_bytes", "ifn_paged_decode",
             "ifn_paged_decode_append", "ifn_paged_decode_planned", "ifn_paged_decode_append_planned",
             "ifn_paged_decode_planning", "ifn_paged_decode_append_planning",
             "ifn_paged_decode_shared_prefix_workspace_bytes", "ifn_paged_decode_shared_prefix",

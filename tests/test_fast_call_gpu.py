@@ -203,3 +203,17 @@ def test_failed_launch_raises_once(dev):
         assert torch.equal(each[0]().view(torch.int16), ref.view(torch.int16))
     finally:
         _fast.load()
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(16, 4, 128), (8, 2, 128), (16, 8, 64), (8, 4, 256)])
+def test_pre_append_shapes_without_a_fused_kernel_are_declined_first(dev, hq, hkv, d):
+    """No output is allocated (or cleared) for a pre-append step that the fused kernel does not cover."""
+    say(f"native pre-append declined hq={hq} hkv={hkv} d={d}")
+    t = _Data(dev, hq=hq, hkv=hkv, d=d)
+    call = lambda fn, **k: fn(t.qf, t.kf, t.vf, t.qw, t.kw, t.rope, t.pos, t.slots, t.act, t.pool, t.table, t.lens, **k)
+    ref = call(kv_prep._qk_norm_rope_store_and_decode)  # (grows the workspace)
+    before = torch.cuda.memory_stats(dev)["allocation.all.allocated"]
+    assert _fast.prep_decode(t.qf, t.kf, t.vf, t.qw, t.kw, t.rope, t.pos, t.slots, t.act, t.pool, t.table, t.lens, 0,
+                             1e-6, None, None, 16, None, None, att._WORKSPACES) is None
+    assert torch.cuda.memory_stats(dev)["allocation.all.allocated"] == before
+    assert torch.equal(call(kv_prep.qk_norm_rope_store_and_decode).view(torch.int16), ref.view(torch.int16))
