@@ -20,32 +20,29 @@
 
 #include <cmath>
 #include <cstdint>
+#include <string>
+#include <type_traits>
 
 #include "../../include/infurnace_amd.h"
 
 namespace {
 
 // The C entry points of the loaded library, by address (bind()).
+#define IFN_ENTRIES(X) \
+  X(store_kv, ifn_store_kv) X(store_kv_layers, ifn_store_kv_layers) \
+  X(decode_ws, ifn_paged_decode_workspace_bytes) X(plan_bytes, ifn_paged_decode_plan_bytes) \
+  X(decode, ifn_paged_decode) X(decode_append, ifn_paged_decode_append) \
+  X(decode_planned, ifn_paged_decode_planned) X(decode_append_planned, ifn_paged_decode_append_planned) \
+  X(decode_planning, ifn_paged_decode_planning) X(decode_append_planning, ifn_paged_decode_append_planning) \
+  X(shared_ws, ifn_paged_decode_shared_prefix_workspace_bytes) X(shared, ifn_paged_decode_shared_prefix) \
+  X(prefill_ws, ifn_paged_prefill_workspace_bytes) X(prefill, ifn_paged_prefill) \
+  X(prefill_append, ifn_paged_prefill_append) X(prep_append, ifn_qk_norm_rope_append) \
+  X(prep_decode, ifn_paged_decode_prep_append) X(prep_decode_planning, ifn_paged_decode_prep_append_planning) \
+  X(prep_prefill, ifn_paged_prefill_prep_append)
 struct Entries {
-  decltype(&ifn_store_kv) store_kv;
-  decltype(&ifn_store_kv_layers) store_kv_layers;
-  decltype(&ifn_paged_decode_workspace_bytes) decode_ws;
-  decltype(&ifn_paged_decode_plan_bytes) plan_bytes;
-  decltype(&ifn_paged_decode) decode;
-  decltype(&ifn_paged_decode_append) decode_append;
-  decltype(&ifn_paged_decode_planned) decode_planned;
-  decltype(&ifn_paged_decode_append_planned) decode_append_planned;
-  decltype(&ifn_paged_decode_planning) decode_planning;
-  decltype(&ifn_paged_decode_append_planning) decode_append_planning;
-  decltype(&ifn_paged_decode_shared_prefix_workspace_bytes) shared_ws;
-  decltype(&ifn_paged_decode_shared_prefix) shared;
-  decltype(&ifn_paged_prefill_workspace_bytes) prefill_ws;
-  decltype(&ifn_paged_prefill) prefill;
-  decltype(&ifn_paged_prefill_append) prefill_append;
-  decltype(&ifn_qk_norm_rope_append) prep_append;
-  decltype(&ifn_paged_decode_prep_append) prep_decode;
-  decltype(&ifn_paged_decode_prep_append_planning) prep_decode_planning;
-  decltype(&ifn_paged_prefill_prep_append) prep_prefill;
+#define IFN_MEMBER(name, fn) decltype(&fn) name;
+  IFN_ENTRIES(IFN_MEMBER)
+#undef IFN_MEMBER
 };
 Entries E{};
 bool bound = false;
@@ -534,20 +531,53 @@ PyObject* guarded(PyObject*, PyObject* const* args, Py_ssize_t n) {
   Py_RETURN_NONE;
 }
 
-PyObject* bind(PyObject*, PyObject* args) {  // the entry points' addresses, in the order of Entries
-  void** at = reinterpret_cast<void**>(&E);
+// The entry points' names and argument kinds in ctypes' letters, as compiled here.
+template <class T>
+constexpr char kind() {
+  if constexpr (std::is_pointer_v<T>) return 'P';
+  else if constexpr (std::is_same_v<T, float>) return 'f';
+  else if constexpr (std::is_same_v<T, size_t>) return 'L';
+  else if constexpr (std::is_same_v<T, int64_t>) return 'l';
+  else {
+    static_assert(std::is_same_v<T, int32_t>);
+    return 'i';
+  }
+}
+template <class R, class... A>
+std::string signature(R (*)(A...)) {
+  return {kind<R>(), kind<A>()...};
+}
+std::string signatures() {
+  std::string all;
+#define IFN_SIGNATURE(name, fn) all += std::string(#fn ":") + signature(decltype(&fn){}) + ",";
+  IFN_ENTRIES(IFN_SIGNATURE)
+#undef IFN_SIGNATURE
+  return all;
+}
+
+// bind(signatures, *addresses): the entry points' addresses, in the order of Entries.  The signatures are those
+// the library was opened with; an extension compiled for others is not bound.
+PyObject* bind(PyObject*, PyObject* args) {
   constexpr Py_ssize_t n = sizeof(Entries) / sizeof(void*);
-  if (PyTuple_GET_SIZE(args) != n) {
-    PyErr_SetString(PyExc_TypeError, "bind: wrong number of entry points");
+  const char* given = PyTuple_GET_SIZE(args) > 0 ? PyUnicode_AsUTF8(PyTuple_GET_ITEM(args, 0)) : nullptr;
+  if (given == nullptr || PyTuple_GET_SIZE(args) != n + 1) {
+    PyErr_SetString(PyExc_TypeError, "bind: the signatures and the entry points' addresses");
     return nullptr;
   }
+  if (signatures() != given) {
+    PyErr_SetString(PyExc_ImportError, "_fast_call was built for other entry points than the library's: rebuild it");
+    return nullptr;
+  }
+  Entries e{};
+  void** at = reinterpret_cast<void**>(&e);
   for (Py_ssize_t i = 0; i < n; ++i) {
-    at[i] = PyLong_AsVoidPtr(PyTuple_GET_ITEM(args, i));
+    at[i] = PyLong_AsVoidPtr(PyTuple_GET_ITEM(args, i + 1));
     if (at[i] == nullptr) {
       if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "bind: null entry point");
       return nullptr;
     }
   }
+  E = e;
   bound = true;
   Py_RETURN_NONE;
 }

@@ -3,13 +3,14 @@
 Each function takes a wrapper's arguments in order, and either makes the call and returns its result (a
 launch that fails raises, as on the Python path) or returns None before the entry point launches anything:
 the arguments are then for the checked Python path, which accepts more forms (array carriers, host values)
-and raises the errors.  Without the extension every call takes that path.
+and raises the errors.  Without a usable extension every call takes that path, after one warning.
 """
 from __future__ import annotations
 
 import ctypes
 import importlib.util
 import os
+import warnings
 
 from .. import _capi
 
@@ -30,13 +31,22 @@ def _none(*args):
     return None
 
 
+def _signature(name):
+    res, args = _capi.SIGNATURES[name]
+    return f"{name}:{''.join(t._type_ for t in (res, *args))},"
+
+
 def load():
-    """The extension, bound to the loaded library's entry points."""
+    """The extension, bound to the loaded library's entry points.
+
+    ImportError when it was compiled for other entry points or signatures than ``_capi`` declares (ctypes'
+    type letters, compared in ``bind``)."""
     lib = _capi.lib()
     spec = importlib.util.spec_from_file_location("_fast_call", EXT_PATH)
     ext = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(ext)
-    ext.bind(*(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in _ENTRIES))
+    ext.bind("".join(map(_signature, _ENTRIES)),
+             *(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in _ENTRIES))
     return ext
 
 
@@ -48,10 +58,10 @@ def _first(name):
             return None  # (the Python path says what is missing)
         try:
             ext = load()
-        except (ImportError, OSError):
-            ext = None
-        for n in _NAMES:
-            globals()[n] = _none if ext is None else getattr(ext, n)
+            globals().update({n: getattr(ext, n) for n in _NAMES})
+        except Exception as e:  # missing, unloadable or stale: no reason to refuse a call
+            globals().update(dict.fromkeys(_NAMES, _none))
+            warnings.warn(f"{EXT_PATH}: {e}; the wrappers' checks run in Python", RuntimeWarning, stacklevel=3)
         return globals()[name](*args)
     return call
 

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 import torch
 
+from infurnace_amd import _capi
 from infurnace_amd.build import CSRC
 from infurnace_amd.kernels import (KVStoreError, PagedAttentionError, _fast, paged_attention, qk_norm_rope_append,
                                    store_kv, store_kv_and_decode)
@@ -56,3 +57,25 @@ def test_device_work_leaves_the_gil():
     work = re.findall(r"at::(?:zeros|empty)\(|\bE\.\w+(?=, )", src)
     out = re.sub(r"(?:unlocked|launch)\((?:[^()]|\((?:[^()]|\([^()]*\))*\))*\)", "", src)
     assert len(work) > 12 and re.findall(r"at::(?:zeros|empty)\(|\bE\.\w+(?=, )", out) == []
+
+
+def test_extension_of_other_signatures_is_not_bound(monkeypatch):
+    """The extension is bound to addresses only where the declared signatures are those it was compiled with."""
+    res, args = _capi.SIGNATURES["ifn_store_kv"]
+    monkeypatch.setitem(_capi.SIGNATURES, "ifn_store_kv", (res, [*args[:1], *args[2:]]))
+    with pytest.raises(ImportError):
+        _fast.load()
+
+
+@pytest.mark.parametrize("error", [ImportError, OSError, TypeError, AttributeError])
+def test_unusable_extension_leaves_the_checked_path(monkeypatch, error):
+    """Missing, stale or unloadable: the wrappers say so once and take their Python path."""
+    def load():
+        raise error("no such extension")
+    monkeypatch.setattr(_fast, "load", load)
+    for n in _fast._NAMES:
+        monkeypatch.setattr(_fast, n, _fast._first(n))
+    with pytest.warns(RuntimeWarning, match="_fast_call"), pytest.raises(KVStoreError):
+        store_kv(POOL, I, None, KV, KV)
+    with pytest.raises(PagedAttentionError):
+        paged_attention(Q, POOL, BT, I)

@@ -192,7 +192,7 @@ def test_failed_launch_raises_once(dev):
             lambda: kv_store.store_kv_layers(t.pool, t.slots, None, torch.stack([t.k] * 2), torch.stack([t.v] * 2))]
     ext = _fast.load()
     try:
-        ext.bind(*at)
+        ext.bind("".join(map(_fast._signature, _fast._ENTRIES)), *at)
         for fn in each:
             del calls[:]
             with pytest.raises(_capi.KernelLaunchError) as e:
