@@ -93,13 +93,19 @@ def sources() -> list[str]:
 
 
 def build(jobs: int = 8) -> str:
-    """Compile all HIP sources for gfx950 and link the shared library; returns its path."""
+    """Compile all HIP sources for gfx950 and link the shared library; returns its path.
+
+    The wrappers' native checks are built beside it where g++ and torch's headers allow; without them the
+    wrappers check in Python, so that is a message and no failure."""
     os.makedirs(BUILD_DIR, exist_ok=True)
     srcs = sources()
     with cf.ThreadPoolExecutor(max_workers=max(1, min(jobs, len(srcs)))) as ex:
         fast = ex.submit(_build_fast)
         objs = list(ex.map(_compile, srcs))
-        fast.result()
+    if fast.exception() is not None:
+        sys.stderr.write(f"fast_call.cpp is not built, the wrappers' checks run in Python: {fast.exception()}\n")
+        if os.path.exists(FAST_PATH):
+            os.remove(FAST_PATH)  # (of an earlier build)
     tmp = LIB_PATH + ".tmp"
     cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs]
     subprocess.run(cmd, check=True)
