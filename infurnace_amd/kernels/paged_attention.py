@@ -167,10 +167,9 @@ def decode_plan(query_shape, kv_pool: torch.Tensor, block_tables: torch.Tensor, 
         return DecodePlan(None, 0, key)
     lib = _capi.lib()
     nbytes = lib.ifn_paged_decode_plan_bytes(n, hq, hkv, d, bs, max_pages, msl)
-    if nbytes == 0:
+    if nbytes == 0 or (sp and hkv * d < 1024):  # (token rows below 2 KiB: their shared-prefix form reads none)
         return DecodePlan(None, 0, key)
-    # (the kernels write every word of a plan; a shared-prefix plan is left alone for some shapes)
-    buf = (torch.zeros if sp else torch.empty)(nbytes, dtype=torch.uint8, device=dev)
+    buf = torch.empty(nbytes, dtype=torch.uint8, device=dev)  # (the kernels write every word of a plan)
 
     def rebuild(slots):
         return decode_plan(query_shape, kv_pool, block_tables, sequence_lengths, active_mask,

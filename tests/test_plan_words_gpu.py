@@ -6,6 +6,7 @@ import torch
 
 from gpu_util import say, to_dev
 from infurnace_amd import _capi
+from infurnace_amd.kernels import decode_plan, paged_attention
 from infurnace_amd.kernels.paged_attention import workspace_for
 from test_decode_planning_gpu import _case
 
@@ -36,3 +37,29 @@ def test_plan_writes_every_word(dev, batch, hi):
                                        ws.numel(), st) == 0
     torch.cuda.synchronize()
     assert torch.equal(bufs[0], bufs[1]) and torch.equal(bufs[0], bufs[2])
+
+
+def test_shared_prefix_plan_words(dev):
+    """The shared-prefix plan of 2 KiB token rows writes every word too; smaller rows, whose shared-prefix decode
+    reads no plan, get an empty one."""
+    say("shared-prefix plan words")
+    rng = np.random.default_rng(6)
+    for hq, hkv, d in ((16, 8, 128), (16, 4, 128), (8, 2, 128), (16, 8, 64)):
+        pool, table, lens, q = _case(rng, [40, 700, 33, 90], hq, hkv, d)
+        table[:, :2] = table[0, :2]
+        qd, p, bt, sl = (to_dev(x, dev) for x in (q, pool, table, lens))
+        pages = bt[0, :2].contiguous()
+        plan = decode_plan(q.shape, p, bt, sl, shared_prefix_pages=pages)
+        out = paged_attention(qd, p, bt, sl, shared_prefix_pages=pages, plan=plan, validate=True)
+        ref = paged_attention(qd, p, bt, sl, shared_prefix_pages=pages)
+        assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+        assert (plan.buf is None) == (hkv * d < 1024)
+        if plan.buf is None:
+            continue
+        L, st = _capi.lib(), torch.cuda.current_stream(dev).cuda_stream
+        for fill in (0xA5, 0xFF):
+            b = torch.full_like(plan.buf, fill)
+            assert L.ifn_paged_decode_shared_prefix_plan(b.data_ptr(), b.numel(), bt.data_ptr(), table.shape[1],
+                                                         sl.data_ptr(), None, 2, p.shape[1], 4, hq, hkv, d, 16,
+                                                         table.shape[1] * 16, st) == 0
+            assert torch.equal(b, plan.buf)
