@@ -9,7 +9,8 @@ import torch
 
 import oracle
 from gpu_util import assert_attn_close, say, to_dev
-from infurnace_amd.kernels import paged_attention, store_kv, store_kv_and_prefill
+from infurnace_amd.kernels import (paged_attention, qk_norm_rope_append, qk_norm_rope_append_and_prefill, rope_table,
+                                   store_kv, store_kv_and_prefill)
 
 pytestmark = pytest.mark.gpu
 
@@ -82,3 +83,23 @@ def test_block_prefill_bad_pages(dev, hq, start, T):
         t2[i, :len(t)] = t
     ref = oracle.paged_attention_rows(q[rows], pool, t2, np.asarray(lens, np.int32))
     assert_attn_close(o2[torch.as_tensor(rows, device=dev)], ref, f"bad pages start={start} T={T}")
+
+
+# one group from 512 workgroups and in 257 .. 511, two groups in 257 .. 511 and 129 .. 256
+@pytest.mark.parametrize("hq,start,T", [(64, 0, 1031), (64, 608, 517), (32, 736, 1100), (64, 288, 272)])
+def test_block_prefill_in_place(dev, hq, start, T):
+    """The pre-append chunk as one call attends in place (its queries lie in the output): equal to the two calls."""
+    say(f"block prefill in place hq={hq} start={start} T={T}")
+    pool, table, q, k, v = _case(hq, 8, start, T)
+    p1, p2, tb, qd, kd, vd = (to_dev(x, dev) for x in (pool, pool, table, q, k, v))
+    g = torch.Generator(device=dev).manual_seed(T)
+    qf, kf, vf = (x.float() + 1e-3 * torch.randn(x.shape, generator=g, device=dev) for x in (qd, kd, vd))
+    w = 1 + 0.1 * torch.randn((2, 128), generator=g, device=dev)
+    rope = rope_table(start + T, 128, 1e6, device=dev)
+    pos = np.arange(start, start + T, dtype=np.int32)
+    slots = (table[pos // 16].astype(np.int64) * 16 + pos % 16).astype(np.int32)
+    q16 = qk_norm_rope_append(qf, kf, vf, w[0], w[1], rope, to_dev(pos, dev), to_dev(slots, dev), None, p1)
+    o1 = paged_attention(q16, p1, tb, None, query_start=start)
+    o2 = qk_norm_rope_append_and_prefill(qf, kf, vf, w[0], w[1], rope, p2, tb, query_start=start)
+    assert torch.equal(p1.view(torch.int16), p2.view(torch.int16)), "pools differ"
+    assert torch.equal(o1.view(torch.int16), o2.view(torch.int16)), "outputs differ"
