@@ -163,10 +163,11 @@ int ifn_paged_decode_append(void* out, const void* query, void* kv_pool_layer, i
  * start each workgroup's page loads one round trip after launch instead of
  * three.  A plan is valid for calls with exactly the inputs it was built
  * from; it holds no pointers, so it may be built on one stream and used on
- * another once ordered after it.  For token rows (num_kv_heads x head_dim fp16)
- * below 2 KiB a missing, short or unaligned plan buffer means no plan rather
- * than an error.  plan_bytes == 0 means these shapes decode
- * without a plan (the planned entry points then ignore it).  slot_mapping may
+ * another once ordered after it; the entry points that build a plan write
+ * every word of it.  For token rows (num_kv_heads x head_dim fp16) below 2 KiB a
+ * missing, short or unaligned plan buffer means no plan rather than an error.
+ * plan_bytes == 0 means these shapes decode without a plan (the planned entry
+ * points then ignore it).  slot_mapping may
  * be NULL for a plan used only by ifn_paged_decode_planned; a plan used by
  * ifn_paged_decode_append_planned must be built with the step's slots (else
  * that call computes the split itself).
@@ -357,9 +358,10 @@ int ifn_paged_decode_shared_prefix_planned(void* out, const void* query, const v
  * fp16) at slot block_table[p / 16] * 16 + p % 16 for p = query_start + t
  * (skipped where that page id is outside the pool, as ifn_store_kv skips
  * such slots), then ifn_paged_prefill(...) on the same stream.  With
- * query_start % 32 == 0 (a multiple of 16 for chunks that fill the chip) this is one launch in which the attention takes the
- * chunk's keys from new_k / new_v; otherwise the store and the attention are
- * two launches.  Same workspace as ifn_paged_prefill.
+ * query_start % 32 == 0 (a multiple of 16 for chunks that fill the chip) this
+ * is one launch in which the attention takes the chunk's keys from new_k /
+ * new_v; otherwise the store and the attention are two launches.  Same
+ * workspace as ifn_paged_prefill.
  * Replaces: store_kv then paged_attention of one prefill chunk
  * (docs/architecture.md:245-246; contiguous form
  * src/infurnace/executor/tinygrad/model.py:116-138).
@@ -452,9 +454,9 @@ int ifn_paged_decode_prep_append(void* out, const float* q, const float* k, cons
 
 /*
  * One prefill chunk of one layer from the fp32 projections, in one call (two
- * launches on the stream): the pre-append of ifn_qk_norm_rope_append (q/k RMSNorm and rotary, k/v cast
- * to fp16 and stored) and the causal attention of ifn_paged_prefill over the
- * result.  Token t of the chunk has position query_start + t, for its rotary
+ * launches on the stream): the pre-append of ifn_qk_norm_rope_append (q/k
+ * RMSNorm and rotary, k/v cast to fp16 and stored) and the causal attention of
+ * ifn_paged_prefill over the result.  Token t of the chunk has position query_start + t, for its rotary
  * angle and for its cache slot block_table[p / 16] * 16 + p % 16 (slots whose
  * page id is outside the pool are not written, and their keys are not
  * attended).  q: fp32 [num_q_tokens][num_q_heads][head_dim]; k, v: fp32
@@ -462,8 +464,8 @@ int ifn_paged_decode_prep_append(void* out, const float* q, const float* k, cons
  * calls.  `out` and the pool are bit-identical to ifn_qk_norm_rope_append(...)
  * with positions query_start + t and those slots, followed by
  * ifn_paged_prefill(...) on the fp16 query.  The fp16 query passes through
- * `out`, which must therefore overlap no other argument.  Requires query_start % 32 == 0 (else IFN_ERR_UNSUPPORTED: run the
- * two calls), query_start + num_q_tokens <= max_positions, every pointer
+ * `out`, which must therefore overlap no other argument.  Requires
+ * query_start % 32 == 0 (else IFN_ERR_UNSUPPORTED: run the two calls), query_start + num_q_tokens <= max_positions, every pointer
  * 16-byte aligned, and the shapes ifn_paged_prefill compiles.  Same workspace
  * as ifn_paged_prefill.
  * Replaces: model.py:109-138 (norm, rope, attention and cache write of a

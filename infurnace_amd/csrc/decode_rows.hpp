@@ -1006,7 +1006,7 @@ __device__ __forceinline__ void decode_rows_body(
       const f16* kb = pool + tok * ROW;
       const f16* vb = pool + v_off + tok * ROW;
       if constexpr (kAppend) {
-        if (ok && tok == slot_b) {  // the appended token (uniform): read it from new_k / new_v
+        if (ok && tok == slot_b) {  // the appended token (uniform when TPW == 1): read it from new_k / new_v
           kb = ap.new_k + int64_t(b) * ROW;
           vb = ap.new_v + int64_t(b) * ROW;
         }

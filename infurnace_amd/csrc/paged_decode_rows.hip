@@ -27,7 +27,7 @@ static RowsKernel pick_rows(int d, int g, int hkv, bool append, bool stream, boo
   }
   // Token rows of 1 KiB and 512 B (tensor-parallel shards of the Qwen3 shapes over 2 and 4 GPUs, 8 x 64):
   // plain and fused-append variants; faster than the per-head kernel at every size measured
-  // (decode_rows.hpp).
+  // (decode_rows.hpp).  Their other groups have not been measured on it and stay on the per-head kernel.
 #define IFN_ROWS_SHARD(DD, GG, HH)                                                                 \
   if (d == DD && g == GG && hkv == HH) {                                                           \
     if (prep || cascade) return nullptr;                                                           \

@@ -14,8 +14,8 @@
 //
 // ifn_paged_prefill_append fuses the chunk's K/V store into the attention launch when
 // query_start is a multiple of 32, or of the page on the block kernel (a key tile, or page, is then
-// wholly before the chunk or wholly in it), and the chunk fits one buffer resource; otherwise store_chunk_kernel stores the rows and the plain attention
-// follows on the same stream, with the same result.
+// wholly before the chunk or wholly in it), and the chunk fits one buffer resource; otherwise
+// store_chunk_kernel stores the rows and the plain attention follows on the same stream, with the same result.
 #include "ifn_common.hpp"
 
 namespace ifn {
@@ -45,7 +45,8 @@ __device__ __forceinline__ void store_chunk_rows(f16* __restrict__ pool, int64_t
   }
 }
 
-// The store alone, for chunks the fused kernel does not take (query_start % 32 != 0).
+// The store alone, for chunks the fused kernels do not take (query_start no multiple of 32, or of the page on the
+// block kernel; chunk rows past one buffer resource).
 __global__ __launch_bounds__(256) void store_chunk_kernel(f16* __restrict__ pool, int64_t num_pages,
                                                           const int32_t* __restrict__ table, int32_t query_start,
                                                           int32_t T, int32_t hkv, int32_t d,

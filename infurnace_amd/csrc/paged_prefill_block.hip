@@ -21,9 +21,10 @@
 //    page to the pool from the registers that carry it to LDS.
 //
 // What bounds it: power, then issue.  2048 queries at 6144, 32 / 8 heads x 128 (240 GFLOP): 275 us,
-// 875 TFLOP/s, against 334 us on the wide kernel (same run); the matrix cores are busy 46% of the cycles
-// and the clock falls to 1.75 GHz (a large fp16 matrix product reaches 1175 TFLOP/s on this card).  8192
-// queries at 0, 16 / 8 heads: 391 -> 308 us.
+// 875 TFLOP/s, against 334 us on the wide kernel (same run).  The matrix cores are busy 46% of the cycles;
+// the clock is 1.87 GHz in the first launches of a burst and falls from there (263 -> 323 us over 12
+// launches in a row; an 8192^3 fp16 product goes from 1355 to 1172 TFLOP/s).  8192 queries at 0, 16 / 8
+// heads: 391 -> 308 us.
 #include "ifn_common.hpp"
 
 namespace ifn {

@@ -4,7 +4,7 @@ pre-append forms, ``decode_plan(..., lazy=True)``).
 The call decodes unplanned and writes, as it goes, the words the plan kernel
 (``ifn_paged_decode_plan``) writes for the same inputs.  Checked here: its output (and pool,
 for the fused forms) equals the unplanned call's bit for bit; the plan it leaves equals the plan
-kernel's byte for byte (both buffers start zeroed); and the later layers' planned calls with it
+kernel's byte for byte (every word of it is written); and the later layers' planned calls with it
 equal the unplanned ones.  Cases cover ragged rows, inactive and empty rows, pages outside the
 pool, ranges holding more pieces than a record describes, calls with fewer ranges than
 workgroups (short batches), 32-token pages and config 2 at full size.
