@@ -521,9 +521,10 @@ def store_kv_and_prefill(query: torch.Tensor, kv_pool: torch.Tensor, block_table
     Same result, in ``out`` and in the pool, as ``store_kv`` of ``new_k``/``new_v`` [T, Hkv, D] at
     the table's slots for positions query_start .. query_start + T - 1 followed by
     ``paged_attention(query, ..., query_start=query_start)`` -- the store of model.py:134-138 and
-    the attention of :116-132.  One launch when query_start % 32 == 0 (16 for chunks that fill
-    the chip), else the store and the attention as two launches.  ``validate``: every table entry the chunk's keys use names a page
-    of the pool (checked before the launch; a debug mode that synchronises).
+    the attention of :116-132.  One launch when query_start % 32 == 0 (% 16 for chunks that
+    fill the chip), else the store and the attention as two launches.  ``validate``: every table entry
+    the chunk's keys use names a page of the pool (checked before the launch; a debug mode that
+    synchronises).
     """
     if not validate and new_k is not None:
         o = _fast.prefill(query, kv_pool, block_table, new_k, new_v, query_start, layer, scale, out, block_size,
