@@ -349,6 +349,30 @@ int prep_chunk_launch(f16* q_out, const PrefillPrep& pp, int32_t max_positions, 
                       const int32_t* block_table, int32_t query_start, int32_t T, int32_t hq, int32_t hkv, int32_t d,
                       int32_t block_size, hipStream_t stream);
 
+typedef __attribute__((address_space(3))) unsigned char lds_u8;
+
+// Transposing LDS read of 4 fp16 per lane (ds_read_b64_tr_b16).  (Device compilation only, like the
+// prefill kernels' other gfx950 builtins: the host pass does not know them and would drop the kernels'
+// launch stubs.)
+__device__ __forceinline__ u32x2 ds_read_tr16(const lds_u8* p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef short v4s __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(
+      u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)(const_cast<lds_u8*>(p))));
+#else
+  return u32x2{0u, 0u};
+#endif
+}
+// Maximum of lanes l and l ^ 32 (v_permlane32_swap: a VALU exchange, no LDS traffic).
+__device__ __forceinline__ float max_lane32(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+#else
+  return x;
+#endif
+}
+
 // Shared-prefix mode of the prefill kernels: every query row sees keys [0, key_len) (no causal
 // mask) and each key split writes its result unnormalised, as the state (m, l, O), for a later
 // merge: ml[((seg * stride + split) * G + g) * 2 + {0,1}], o[((seg * stride + split) * G + g) * D + dim]

@@ -36,7 +36,6 @@ constexpr int kBWaves = 4;
 constexpr int kBThreads = kBWaves * kWave;
 constexpr int kBXcdCus = 32;             // CUs per XCD, 8 XCDs
 
-typedef __attribute__((address_space(3))) unsigned char lds_u8;
 typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
 
 template <int D, int G>
@@ -60,23 +59,6 @@ struct BlockCfg {
   static_assert(kQw % kBPage == 0, "a workgroup's queries are whole pages of the chunk");
 };
 
-__device__ __forceinline__ u32x2 blk_read_tr16(const lds_u8* p) {  // ds_read_b64_tr_b16
-#if defined(__HIP_DEVICE_COMPILE__)
-  typedef short v4s __attribute__((ext_vector_type(4)));
-  return __builtin_bit_cast(
-      u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)(const_cast<lds_u8*>(p))));
-#else
-  return u32x2{0u, 0u};
-#endif
-}
-__device__ __forceinline__ float blk_max_lane32(float x) {  // maximum of lanes l and l ^ 32
-#if defined(__HIP_DEVICE_COMPILE__)
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-#else
-  return x;
-#endif
-}
 // No instruction: the values must exist at this point.
 __device__ __forceinline__ void blk_pin(f16x8& a, f16x8& b) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -272,7 +254,7 @@ __global__ __launch_bounds__(KS * kBThreads, 2) void prefill_block_kernel(
       const int o = 4 * (a % 4);
       mx[a] = fmaxf(fmaxf(x[o], x[o + 1]), fmaxf(x[o + 2], x[o + 3]));
     }
-    cand = blk_max_lane32(fmaxf(fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3])),
+    cand = max_lane32(fmaxf(fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3])),
                                 fmaxf(fmaxf(mx[4], mx[5]), fmaxf(mx[6], mx[7])))) * scale_log2;
   };
   // Lazy rescale: the reference maximum moves only when a score exceeds it by more than 8 (log2
@@ -305,8 +287,8 @@ __global__ __launch_bounds__(KS * kBThreads, 2) void prefill_block_kernel(
 #pragma unroll
     for (int dt = 0; dt < kDT; ++dt) {
       const lds_u8* a = b + vfrag + u * kBPage * C::kVRowB + 64 * dt;
-      const f16x4 lo = __builtin_bit_cast(f16x4, blk_read_tr16(a));
-      const f16x4 hi = __builtin_bit_cast(f16x4, blk_read_tr16(a + 8 * C::kVRowB));
+      const f16x4 lo = __builtin_bit_cast(f16x4, ds_read_tr16(a));
+      const f16x4 hi = __builtin_bit_cast(f16x4, ds_read_tr16(a + 8 * C::kVRowB));
       const f16x8 vf = f16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
       acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, p, acc[dt], 0, 0, 0);
     }

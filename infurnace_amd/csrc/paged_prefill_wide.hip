@@ -153,32 +153,9 @@ __device__ __forceinline__ void wide_store_chunk(f16* __restrict__ pool, int64_t
   }
 }
 
-typedef __attribute__((address_space(3))) unsigned char lds_u8;
-
-// Transposing LDS read of 4 fp16 per lane (ds_read_b64_tr_b16).  (Device compilation only, like the
-// other gfx950 builtins below: the host pass does not know them and would drop the kernels' launch
-// stubs.)
-__device__ __forceinline__ u32x2 ds_read_tr16(const lds_u8* p) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  typedef short v4s __attribute__((ext_vector_type(4)));
-  return __builtin_bit_cast(
-      u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)(const_cast<lds_u8*>(p))));
-#else
-  return u32x2{0u, 0u};
-#endif
-}
 // 16-byte buffer load (buffer_load_dwordx4); an offset past the resource's end reads zeros.
 __device__ __forceinline__ u32x4 buf_ld16(__amdgpu_buffer_rsrc_t r, uint32_t off) {
   return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
-}
-// Maximum of lanes l and l ^ 32 (v_permlane32_swap: a VALU exchange, no LDS traffic).
-__device__ __forceinline__ float max_lane32(float x) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-#else
-  return x;
-#endif
 }
 // No instruction: the value is held in accumulation registers from here on (the queries, read
 // only as MFMA operands, which take them from there without copies).
